@@ -120,7 +120,7 @@ struct Cells
 	int off[3], dim[3];
 	double begin[3], end[3];
 	int enabled[3];
-	DBuf start, atoms;
+	DBuf start, rec32, rec64; // list starts, the lists' records
 };
 
 struct Receptor
@@ -775,9 +775,16 @@ Cells& receptor_cells(sgpu_ctx* c, Receptor& r, const sgpu_grid_dims& gd)
 	int total = 0;
 	hip_check(hipMemcpyAsync(&total, a.cell_start + ncells, sizeof(int), hipMemcpyDeviceToHost, c->stream), "cells");
 	hip_check(hipStreamSynchronize(c->stream), "cells");
-	cl->atoms.alloc(size_t(std::max(1, total)) * sizeof(int));
-	a.cell_atoms = cl->atoms.as<int>();
+	// both precisions: any later call with this box finds its records
+	DBuf atoms;
+	atoms.alloc(size_t(std::max(1, total)) * sizeof(int));
+	cl->rec32.alloc(size_t(std::max(1, total)) * sizeof(RecAtom<float>));
+	cl->rec64.alloc(size_t(std::max(1, total)) * sizeof(RecAtom<double>));
+	a.cell_atoms = atoms.as<int>();
 	hip_check(launch_cell_fill(a, c->stream), "cell fill");
+	hip_check(launch_cell_records(a.rec_xyz, a.rec_type, a.cell_atoms, total, cl->rec32.as<RecAtom<float>>(),
+					  cl->rec64.as<RecAtom<double>>(), c->stream),
+			"cell records");
 	hip_check(hipStreamSynchronize(c->stream), "cells");
 	Cells& ref = *cl;
 	r.cells[key] = std::move(cl);
@@ -793,7 +800,7 @@ ReceptorPtrs<T> receptor_ptrs(const Receptor& r, const Cells& cl)
 	p.charge = (sizeof(T) == 8 ? r.q64 : r.q32).template as<T>();
 	p.natoms = r.n;
 	p.cell_start = cl.start.as<int>();
-	p.cell_atoms = cl.atoms.as<int>();
+	p.cell_recs = (sizeof(T) == 8 ? cl.rec64 : cl.rec32).template as<RecAtom<T>>();
 	for (int d = 0; d < 3; d++)
 	{
 		p.cell_off[d] = cl.off[d];

@@ -131,6 +131,18 @@ __global__ __launch_bounds__(CELL_THREADS) void cell_fill_kernel(GridBuildArgs a
 	}
 }
 
+__global__ __launch_bounds__(256) void cell_records_kernel(const double* xyz, const int* type, const int* cell_atoms,
+		int total, RecAtom<float>* rec32, RecAtom<double>* rec64)
+{
+	const int k = int(blockIdx.x * blockDim.x + threadIdx.x);
+	if (k >= total)
+		return;
+	const int i = cell_atoms[k];
+	const double x = xyz[3 * size_t(i)], y = xyz[3 * size_t(i) + 1], z = xyz[3 * size_t(i) + 2];
+	rec64[k] = make_rec_atom<double>(x, y, z, type[i], i);
+	rec32[k] = make_rec_atom<float>(float(x), float(y), float(z), type[i], i);
+}
+
 __global__ __launch_bounds__(256) void grid_points_kernel(GridBuildArgs a, double* points, double* qpoints)
 {
 	const size_t npts = size_t(a.dim[0]) * a.dim[1] * a.dim[2];
@@ -253,6 +265,16 @@ hipError_t launch_cell_fill(const GridBuildArgs& a, hipStream_t st)
 {
 	const int ncells = a.cell_dim[0] * a.cell_dim[1] * a.cell_dim[2];
 	hipLaunchKernelGGL(cell_fill_kernel, dim3(ncells), dim3(CELL_THREADS), 0, st, a);
+	return hipGetLastError();
+}
+
+hipError_t launch_cell_records(const double* xyz, const int* type, const int* cell_atoms, int total,
+		RecAtom<float>* rec32, RecAtom<double>* rec64, hipStream_t st)
+{
+	if (total < 1)
+		return hipSuccess;
+	hipLaunchKernelGGL(cell_records_kernel, dim3(unsigned((total + 255) / 256)), dim3(256), 0, st, xyz, type,
+			cell_atoms, total, rec32, rec64);
 	return hipGetLastError();
 }
 

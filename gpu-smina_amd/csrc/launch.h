@@ -143,6 +143,9 @@ struct GridBuildArgs
 };
 hipError_t launch_cell_count(const GridBuildArgs& a, hipStream_t st);
 hipError_t launch_cell_fill(const GridBuildArgs& a, hipStream_t st);
+// the list entries of every cell as records, in both precisions
+hipError_t launch_cell_records(const double* xyz, const int* type, const int* cell_atoms, int total,
+		RecAtom<float>* rec32, RecAtom<double>* rec64, hipStream_t st);
 // points: [ntypes][npts]; qpoints: the charge maps, same layout (ncomp 4)
 hipError_t launch_grid_points(const GridBuildArgs& a, double* points, double* qpoints, hipStream_t st);
 template<typename T>

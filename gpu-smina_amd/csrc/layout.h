@@ -149,6 +149,29 @@ struct GridPtrs
 	double slope;
 };
 
+// one entry of a cell's list of receptor atoms, in one 16-byte (FP32) or
+// 32-byte (FP64) record: position, type (5 bits) and receptor index (the
+// rest), so that a lane reads an atom with one aligned load and the entries
+// of a list follow each other
+template<typename T> struct RecMeta;
+template<> struct RecMeta<float> { using type = unsigned; };
+template<> struct RecMeta<double> { using type = unsigned long long; };
+template<typename T>
+struct alignas(4 * sizeof(T)) RecAtom
+{
+	T x, y, z;
+	typename RecMeta<T>::type meta;
+};
+template<typename T>
+__host__ __device__ inline RecAtom<T> make_rec_atom(T x, T y, T z, int type, int index)
+{
+	return {x, y, z, typename RecMeta<T>::type(unsigned(type) | (unsigned(index) << 5))};
+}
+template<typename T>
+__host__ __device__ inline int rec_type(const RecAtom<T>& a) { return int(unsigned(a.meta) & 31u); }
+template<typename T>
+__host__ __device__ inline int rec_index(const RecAtom<T>& a) { return int(unsigned(a.meta) >> 5); }
+
 // receptor for the direct (non_cache) back end: atoms and 3 A cells over
 // the box holding, in receptor order, the atoms within the cutoff of the
 // cell's brick
@@ -160,7 +183,7 @@ struct ReceptorPtrs
 	const T* charge;     // [natoms] partial charges
 	int natoms;
 	const int* cell_start; // [ncells+1]
-	const int* cell_atoms;
+	const RecAtom<T>* cell_recs;
 	int cell_off[3];
 	int cell_dim[3];
 	double begin[3];

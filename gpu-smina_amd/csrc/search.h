@@ -41,6 +41,8 @@ namespace sgpu
 constexpr int PAIR_BATCH = 4;
 // list entries per batch of the FP32 per-atom pair-force gather
 constexpr int GATHER_BATCH = 4;
+// receptor atoms per batch of the direct term
+constexpr int REC_BATCH = 4;
 // the unordered search evaluates each pair once, pair-parallel, and sums
 // each atom's pair forces from LDS; the ordered one walks each atom's
 // neighbour list in smina's order, evaluating every pair from both ends
@@ -564,25 +566,93 @@ __device__ inline T direct_term(const EvalCtx<T>& ec, int t1, T q1, V3<T> ac, V3
 	T this_e = 0;
 	V3<T> deriv = v3(T(0), T(0), T(0));
 	const V3<T> adjv = v3(adj[0], adj[1], adj[2]);
-	for (int k = r.cell_start[cell]; k < r.cell_start[cell + 1]; k++)
+	// The list in batches of REC_BATCH, accumulated in list order: the next
+	// batch's records are loaded ahead and a batch's table rows are in flight
+	// together (an entry out of range reads row 0 and is skipped).  The loop
+	// is bound by the latency of these dependent loads, not by their bytes:
+	// one entry at a time (index, position, type, row, each waited for) took
+	// 330 ms against 121 ms for the FP32 refinement of the 1,024-ligand
+	// screen's saved poses, and 230 ms against 160 ms for the FP64 refinement
+	// of 256 parsed poses with splines.
+	const int k0 = r.cell_start[cell], k1 = r.cell_start[cell + 1];
+	RecAtom<T> next[REC_BATCH];
+#pragma unroll
+	for (int u = 0; u < REC_BATCH; u++)
+		next[u] = r.cell_recs[k0 + u < k1 ? k0 + u : 0];
+	for (int k = k0; k < k1; k += REC_BATCH)
 	{
-		const int j = r.cell_atoms[k];
-		const V3<T> rba = adjv - ld3(r.xyz + 3 * j);
-		const T r2 = norm_sqr(rba);
-		if (r2 < T(ec.tab.cutoff_sqr))
+		V3<T> rba[REC_BATCH];
+		T r2[REC_BATCH], pe[REC_BATCH], pd[REC_BATCH];
+		int type[REC_BATCH], idx[REC_BATCH];
+		bool ok[REC_BATCH];
+#pragma unroll
+		for (int u = 0; u < REC_BATCH; u++)
 		{
-			if (r2 < Real<T>::eps())
-				atomicOr(ec.error, 1); // bit 0: exact overlap (other bits belong to the caller)
-			T pe, pd;
-			if (ec.tab.ncomp == 4)
-				table_deriv_charged(ec.tab, t1, r.type[j], q1, r.charge[j], r2, pe, pd);
-			else
-				table_deriv(ec.tab, tri_index_permissive(t1, r.type[j]), r2, pe, pd);
-			this_e += pe;
-			deriv.x += pd * rba.x;
-			deriv.y += pd * rba.y;
-			deriv.z += pd * rba.z;
+			rba[u] = adjv - v3(next[u].x, next[u].y, next[u].z);
+			r2[u] = norm_sqr(rba[u]);
+			ok[u] = k + u < k1 && r2[u] < T(ec.tab.cutoff_sqr);
+			type[u] = rec_type(next[u]);
+			idx[u] = rec_index(next[u]);
 		}
+#pragma unroll
+		for (int u = 0; u < REC_BATCH; u++)
+			next[u] = r.cell_recs[k + REC_BATCH + u < k1 ? k + REC_BATCH + u : 0];
+		if (ec.tab.kind == 1)
+		{
+			SplineRow row[REC_BATCH];
+#pragma unroll
+			for (int u = 0; u < REC_BATCH; u++)
+				row[u] = spline_row(ec.tab.spl, ec.tab.spl_cut, ec.tab.fraction, ec.tab.nseg,
+						tri_index_permissive(t1, type[u]), __builtin_sqrt(double(ok[u] ? r2[u] : T(0))));
+#pragma unroll
+			for (int u = 0; u < REC_BATCH; u++)
+			{
+				double val, der;
+				spline_value(row[u], val, der);
+				pe[u] = T(val);
+				pd[u] = T(der / row[u].r);
+			}
+		}
+		else if (ec.tab.ncomp == 4)
+		{
+#pragma unroll
+			for (int u = 0; u < REC_BATCH; u++)
+				table_deriv_charged(ec.tab, t1, type[u], q1, r.charge[ok[u] ? idx[u] : 0], ok[u] ? r2[u] : T(0), pe[u],
+						pd[u]);
+		}
+		else
+		{
+			T e1[REC_BATCH], d1[REC_BATCH], e2[REC_BATCH], d2[REC_BATCH], rem[REC_BATCH];
+#pragma unroll
+			for (int u = 0; u < REC_BATCH; u++)
+			{
+				const T r2f = T(ec.tab.factor) * r2[u];
+				const int i1 = ok[u] ? int(r2f) : 0;
+				rem[u] = r2f - T(i1);
+				const T* p = ec.tab.smooth + (ok[u] ? size_t(tri_index_permissive(t1, type[u])) * ec.tab.n + i1 : 0) * 2;
+				e1[u] = p[0];
+				d1[u] = p[1];
+				e2[u] = p[2];
+				d2[u] = p[3];
+			}
+#pragma unroll
+			for (int u = 0; u < REC_BATCH; u++)
+			{
+				pe[u] = e1[u] + rem[u] * (e2[u] - e1[u]);
+				pd[u] = d1[u] + rem[u] * (d2[u] - d1[u]);
+			}
+		}
+#pragma unroll
+		for (int u = 0; u < REC_BATCH; u++)
+			if (ok[u])
+			{
+				if (r2[u] < Real<T>::eps())
+					atomicOr(ec.error, 1); // bit 0: exact overlap (other bits belong to the caller)
+				this_e += pe[u];
+				deriv.x += pd[u] * rba[u].x;
+				deriv.y += pd[u] * rba[u].y;
+				deriv.z += pd[u] * rba[u].z;
+			}
 	}
 	// the user grid at the atom's own position, with the back end's slope
 	V3<T> ug_deriv = v3(T(0), T(0), T(0));
