@@ -154,9 +154,10 @@ struct Grid
 struct HostBatch
 {
 	std::vector<ModelHdr> hdr;
-	std::vector<int> iblob, pair_a, pair_b, pair_tri;
+	std::vector<int> iblob;
 	std::vector<double> tblob;
 	WavePlan plan{};
+	WavePlan limit{}; // the sizes that admit a model (limit_bytes)
 };
 
 struct Batch
@@ -164,7 +165,7 @@ struct Batch
 	int precision = 0;
 	int n = 0;
 	HostBatch h;
-	DBuf hdr, iblob, tblob, pair_a, pair_b, pair_tri;
+	DBuf hdr, iblob, tblob;
 	// FP64 copy for the final rescoring when the batch searches in FP32
 	std::unique_ptr<Batch> fp64;
 };
@@ -253,6 +254,9 @@ struct sgpu_ctx
 namespace
 {
 
+constexpr int LDS_LIMIT = 160 * 1024;
+constexpr int LDS_STATIC = 64; // the persistent Monte Carlo kernel's own LDS (its work item)
+
 // the LDS plan that fits every listed model of a packed batch
 WavePlan plan_for(const HostBatch& B, const std::vector<int>& models)
 {
@@ -281,6 +285,9 @@ WavePlan plan_for(const HostBatch& B, const std::vector<int>& models)
 	p.tmax = tmax;
 	p.amax = amax;
 	p.bytes = 0;
+	// FP64: the pairs' factors in LDS unless one chain would not fit with them
+	p.pair_lds = 1;
+	p.pair_lds = block_lds_bytes<double>(p, 1) + LDS_STATIC <= LDS_LIMIT ? 1 : 0;
 	return p;
 }
 
@@ -312,15 +319,6 @@ void pack_batch(const sgpu_flat_model* ms, int n, HostBatch& B)
 		std::vector<int> I;
 		std::vector<double> R;
 		auto mark = [&](int& off) { off = int(I.size()); };
-		// atoms
-		mark(h.o_type);
-		I.insert(I.end(), m.atom_type, m.atom_type + na);
-		mark(h.o_afr);
-		for (int i = 0; i < m.natoms; i++)
-		{
-			require(m.atom_frame[i] >= 0 && m.atom_frame[i] < m.nframes, "atom frame out of range");
-			I.push_back(m.atom_frame[i]);
-		}
 		// neighbour lists in evaluation (pair) order
 		std::vector<std::vector<int>> lists(m.natoms);
 		for (int p = 0; p < m.npairs; p++)
@@ -330,30 +328,37 @@ void pack_batch(const sgpu_flat_model* ms, int n, HostBatch& B)
 			const int tri = m.pair_tri[p];
 			require(tri >= 0 && tri < SGPU_NUM_TYPE_PAIRS, "pair type index out of range");
 			require(tri == tri_index_permissive(m.atom_type[a], m.atom_type[b]), "pair table index disagrees with types");
-			const bool other = p < m.nother;
-			lists[a].push_back(make_code(b, tri, false, other, p));
+			lists[a].push_back(make_code(b, p + 1));
 			if (b < m.natoms)
-				lists[b].push_back(make_code(a, tri, true, other, p));
+				lists[b].push_back(make_code(a, p + 1));
 		}
-		mark(h.o_nbr);
-		int k = 0;
+		int nlisted = 0;
 		for (int i = 0; i < m.natoms; i++)
 		{
-			I.push_back(k);
-			k += int(lists[i].size());
+			nlisted += int(lists[i].size());
+			while (lists[i].size() % NBR_BATCH)
+				lists[i].push_back(make_code(i, 0));
 		}
-		I.push_back(k);
+		// the movable atoms' records, first in the blob (stage_model)
+		int ncodes = 0;
+		for (int i = 0; i < m.natoms; i++)
+		{
+			require(m.atom_frame[i] >= 0 && m.atom_frame[i] < m.nframes, "atom frame out of range");
+			I.push_back(make_atom(m.atom_frame[i], m.atom_type[i], !is_hydrogen_type(m.atom_type[i])));
+			const int end = ncodes + int(lists[i].size());
+			I.push_back(int(unsigned(ncodes) | (unsigned(end) << 16)));
+			ncodes = end;
+		}
+		mark(h.o_type);
+		I.insert(I.end(), m.atom_type, m.atom_type + na);
+		I.resize((I.size() + 3) / 4 * 4, 0); // codes are read 16 bytes at a time
 		mark(h.o_code);
+		h.ncodes = ncodes;
 		for (int i = 0; i < m.natoms; i++)
 			I.insert(I.end(), lists[i].begin(), lists[i].end());
-		if (I.size() % 2)
-			I.push_back(0); // pair records are read as 8-byte words
 		mark(h.o_prec);
 		for (int p = 0; p < m.npairs; p++)
-		{
-			I.push_back(int(unsigned(3 * m.pair_a[p]) | (unsigned(3 * m.pair_b[p]) << 16)));
-			I.push_back(int(unsigned(m.pair_tri[p]) | (unsigned(p < m.nother) << 16)));
-		}
+			I.push_back(make_prec(m.pair_a[p], m.pair_b[p], m.pair_tri[p]));
 		// frames, children, levels
 		std::vector<int> depth(m.nframes, 0);
 		int nlevels = 0;
@@ -369,18 +374,6 @@ void pack_batch(const sgpu_flat_model* ms, int n, HostBatch& B)
 			require((m.frame_kind[f] == SGPU_FRAME_SEGMENT) == (p >= 0), "only segments have parents");
 		}
 		h.nlevels = nlevels;
-		mark(h.o_fparent);
-		I.insert(I.end(), m.frame_parent, m.frame_parent + m.nframes);
-		mark(h.o_fkind);
-		I.insert(I.end(), m.frame_kind, m.frame_kind + m.nframes);
-		mark(h.o_fbegin);
-		I.insert(I.end(), m.frame_begin, m.frame_begin + m.nframes);
-		mark(h.o_fend);
-		I.insert(I.end(), m.frame_end, m.frame_end + m.nframes);
-		mark(h.o_fconf);
-		I.insert(I.end(), m.frame_conf, m.frame_conf + m.nframes);
-		mark(h.o_fchange);
-		I.insert(I.end(), m.frame_change, m.frame_change + m.nframes);
 		// end of each frame's subtree atoms: a subtree is a run of frames in
 		// preorder whose atom ranges follow each other
 		std::vector<int> send(m.frame_end, m.frame_end + m.nframes);
@@ -389,18 +382,22 @@ void pack_batch(const sgpu_flat_model* ms, int n, HostBatch& B)
 				send[size_t(m.frame_parent[f])] = std::max(send[size_t(m.frame_parent[f])], send[size_t(f)]);
 		for (int f = 0; f + 1 < m.nframes; f++)
 			require(m.frame_end[f] == m.frame_begin[f + 1], "frame atom ranges must follow preorder");
-		mark(h.o_fsend);
-		I.insert(I.end(), send.begin(), send.end());
-		// each frame's path from its tree root (frame indices as bytes, root
-		// first, the frame itself last) for the ancestor walk of set_conf
-		mark(h.o_fdepth);
+		if (I.size() % 2)
+			I.push_back(0); // frame records are read as 8-byte words
+		mark(h.o_fm);
 		h.path_ok = 1;
 		for (int f = 0; f < m.nframes; f++)
 		{
-			I.push_back(depth[size_t(f)] + 1);
+			const int ci = m.frame_conf[f], gi = m.frame_change[f];
+			require(ci >= 0 && ci < m.conf_size && gi >= 0 && gi < m.change_size, "frame conf index out of range");
+			I.push_back(make_frame0(m.frame_kind[f], ci, gi, depth[size_t(f)]));
+			I.push_back(make_frame1(m.frame_begin[f], send[size_t(f)], m.frame_end[f],
+					m.frame_parent[f] < 0 ? 255 : m.frame_parent[f]));
 			if (depth[size_t(f)] + 1 > MAX_PATH)
 				h.path_ok = 0;
 		}
+		// each frame's path from its tree root (frame indices as bytes, root
+		// first, the frame itself last) for the ancestor walk of set_conf
 		mark(h.o_fpath);
 		for (int f = 0; f < m.nframes; f++)
 		{
@@ -413,37 +410,18 @@ void pack_batch(const sgpu_flat_model* ms, int n, HostBatch& B)
 				I.push_back(int(unsigned(path[size_t(4 * w)]) | (unsigned(path[size_t(4 * w + 1)]) << 8) |
 						(unsigned(path[size_t(4 * w + 2)]) << 16) | (unsigned(path[size_t(4 * w + 3)]) << 24)));
 		}
-		std::vector<int> cstart, ccount, clist;
+		std::vector<int> clist;
+		mark(h.o_child);
 		for (int f = 0; f < m.nframes; f++)
 		{
-			cstart.push_back(int(clist.size()));
-			int cnt = 0;
+			const int start = int(clist.size());
 			for (int c = f + 1; c < m.nframes; c++)
 				if (m.frame_parent[c] == f)
-				{
 					clist.push_back(c);
-					++cnt;
-				}
-			ccount.push_back(cnt);
+			I.push_back(make_child(start, int(clist.size()) - start));
 		}
-		mark(h.o_cstart);
-		I.insert(I.end(), cstart.begin(), cstart.end());
-		mark(h.o_ccount);
-		I.insert(I.end(), ccount.begin(), ccount.end());
 		mark(h.o_clist);
 		I.insert(I.end(), clist.begin(), clist.end());
-		mark(h.o_lstart);
-		std::vector<int> lframes;
-		for (int L = 0; L < nlevels; L++)
-		{
-			I.push_back(int(lframes.size()));
-			for (int f = 0; f < m.nframes; f++)
-				if (depth[f] == L)
-					lframes.push_back(f);
-		}
-		I.push_back(int(lframes.size()));
-		mark(h.o_lframes);
-		I.insert(I.end(), lframes.begin(), lframes.end());
 		// heavy atoms
 		mark(h.o_heavy);
 		int nh = 0;
@@ -488,24 +466,18 @@ void pack_batch(const sgpu_flat_model* ms, int n, HostBatch& B)
 			tpb[t] = pb;
 			tpe[t] = pe;
 		}
-		mark(h.o_troot);
-		I.insert(I.end(), troot.begin(), troot.end());
-		mark(h.o_tconf);
-		I.insert(I.end(), tconf.begin(), tconf.end());
-		mark(h.o_tchange);
-		I.insert(I.end(), tchg.begin(), tchg.end());
-		mark(h.o_tlig);
-		I.insert(I.end(), tlig.begin(), tlig.end());
-		mark(h.o_tntors);
-		I.insert(I.end(), tn.begin(), tn.end());
-		mark(h.o_tab);
-		I.insert(I.end(), tab.begin(), tab.end());
-		mark(h.o_tae);
-		I.insert(I.end(), tae.begin(), tae.end());
-		mark(h.o_tpb);
-		I.insert(I.end(), tpb.begin(), tpb.end());
-		mark(h.o_tpe);
-		I.insert(I.end(), tpe.begin(), tpe.end());
+		mark(h.o_tree);
+		int nlig = 0;
+		h.one_ligand = 1;
+		for (int t = 0; t < m.ntrees; t++)
+		{
+			I.insert(I.end(), {troot[t], tconf[t], tchg[t], tlig[t], tn[t], tab[t], tae[t], tpb[t], tpe[t]});
+			nlig += tlig[t];
+			if (tlig[t] && m.npairs > m.nother && (tpb[t] != m.nother || tpe[t] != m.npairs))
+				h.one_ligand = 0;
+		}
+		if (nlig > 1 || (nlig == 0 && m.npairs > m.nother))
+			h.one_ligand = 0;
 		// conf / change maps
 		std::vector<int> ck(m.conf_size, -1), cc(m.conf_size, 0), gk(m.change_size, -1), gc(m.change_size, 0);
 		for (int f = 0; f < m.nframes; f++)
@@ -546,36 +518,46 @@ void pack_batch(const sgpu_flat_model* ms, int n, HostBatch& B)
 			require(v >= 0, "conf element without a frame");
 		for (int v : gk)
 			require(v >= 0, "change element without a frame");
-		mark(h.o_maps);
-		I.insert(I.end(), ck.begin(), ck.end());
-		I.insert(I.end(), cc.begin(), cc.end());
-		I.insert(I.end(), gk.begin(), gk.end());
-		I.insert(I.end(), gc.begin(), gc.end());
-		// reals
+		mark(h.o_cmap);
+		for (int k = 0; k < m.conf_size; k++)
+			I.push_back(make_map(ck[size_t(k)], cc[size_t(k)]));
+		mark(h.o_gmap);
+		for (int k = 0; k < m.change_size; k++)
+			I.push_back(make_map(gk[size_t(k)], gc[size_t(k)]));
+		// reals; records of 4 are read 16 bytes at a time
+		auto align4 = [&]() { R.resize((R.size() + 3) / 4 * 4, 0.0); };
+		auto records = [&](const double* src, int count) {
+			for (int k = 0; k < count; k++)
+				R.insert(R.end(), {src[3 * k], src[3 * k + 1], src[3 * k + 2], 0.0});
+		};
 		h.o_xyz0 = int(R.size());
 		R.insert(R.end(), m.atom_init, m.atom_init + 3 * na);
+		align4();
 		h.o_local = int(R.size());
-		R.insert(R.end(), m.atom_local, m.atom_local + 3 * m.natoms);
+		records(m.atom_local, m.natoms);
 		h.o_forig = int(R.size());
-		R.insert(R.end(), m.frame_origin, m.frame_origin + 3 * m.nframes);
+		records(m.frame_origin, m.nframes);
 		h.o_faxis = int(R.size());
-		R.insert(R.end(), m.frame_axis, m.frame_axis + 3 * m.nframes);
+		records(m.frame_axis, m.nframes);
 		h.o_charge = int(R.size());
 		if (m.atom_charge)
 			R.insert(R.end(), m.atom_charge, m.atom_charge + na);
 		else
 			R.insert(R.end(), size_t(na), 0.0);
+		// the sizes that admit a model to a workgroup's LDS (limit_bytes):
+		// one word or real per array element, as limits stated for this ABI
+		const int words = (na + 2 * m.natoms + 1 + nlisted + 1) / 2 * 2 + 2 * m.npairs +
+				m.nframes * (11 + MAX_PATH / 4) + int(clist.size()) + nlevels + 1 + nh + 9 * m.ntrees +
+				2 * m.conf_size + 2 * m.change_size;
+		B.limit.imax = std::max(B.limit.imax, words);
+		B.limit.tmax = std::max(B.limit.tmax, 4 * na + 3 * m.natoms + 6 * m.nframes);
 		// append
 		h.iblob_off = int(B.iblob.size());
 		h.iblob_len = int(I.size());
 		h.tblob_off = int(B.tblob.size());
 		h.tblob_len = int(R.size());
-		h.pair_off = int(B.pair_a.size());
 		B.iblob.insert(B.iblob.end(), I.begin(), I.end());
 		B.tblob.insert(B.tblob.end(), R.begin(), R.end());
-		B.pair_a.insert(B.pair_a.end(), m.pair_a, m.pair_a + m.npairs);
-		B.pair_b.insert(B.pair_b.end(), m.pair_b, m.pair_b + m.npairs);
-		B.pair_tri.insert(B.pair_tri.end(), m.pair_tri, m.pair_tri + m.npairs);
 		B.hdr.push_back(h);
 	}
 	std::vector<int> all(static_cast<size_t>(n));
@@ -596,9 +578,6 @@ void upload_batch(Batch& b, hipStream_t st)
 	b.hdr.alloc(h.hdr.size() * sizeof(ModelHdr));
 	hip_check(hipMemcpyAsync(b.hdr.p, h.hdr.data(), h.hdr.size() * sizeof(ModelHdr), hipMemcpyHostToDevice, st), "hdr");
 	upload(b.iblob, h.iblob, st);
-	upload(b.pair_a, h.pair_a, st);
-	upload(b.pair_b, h.pair_b, st);
-	upload(b.pair_tri, h.pair_tri, st);
 	if (b.precision == SGPU_FP64)
 		upload(b.tblob, h.tblob, st);
 	else
@@ -613,9 +592,6 @@ BatchPtrs<T> ptrs(const Batch& b)
 	p.hdr = b.hdr.as<ModelHdr>();
 	p.iblob = b.iblob.as<int>();
 	p.tblob = b.tblob.as<T>();
-	p.pair_a = b.pair_a.as<int>();
-	p.pair_b = b.pair_b.as<int>();
-	p.pair_tri = b.pair_tri.as<int>();
 	return p;
 }
 
@@ -625,10 +601,20 @@ int plan_bytes(const WavePlan& p, int prec, int waves)
 	       : prec == SGPU_MIXED ? block_lds_bytes<float, double>(p, waves)
 	                            : block_lds_bytes<float>(p, waves);
 }
+// The size a model may have: the LDS of one chain of it in a layout of one
+// word or real per element, with a force per pair in FP32.  The layout in use
+// needs less for every model near the limit; the limit itself stays.
+int limit_bytes(const WavePlan& p, const WavePlan& limit, int prec)
+{
+	const int t = prec == SGPU_FP64 ? 8 : 4, s = prec == SGPU_FP32 ? 4 : 8;
+	const int eval = 3 * p.amax + 4 * p.nmax + 25 * p.fmax + p.gmax + p.cmax +
+			(prec == SGPU_FP64 ? 0 : 3 * std::max(p.pmax, p.nmax));
+	const int search = p.gmax + p.hmax + (s != t ? p.cmax + p.gmax : 0);
+	auto up = [](int bytes) { return (bytes + 15) / 16 * 16; };
+	return up((limit.imax + p.amax) * 4) + up(limit.tmax * t) + up(eval * t) + up(search * s);
+}
 // the precision of a batch's model evaluation (and so of its maps)
 int eval_precision(int prec) { return prec == SGPU_FP64 ? SGPU_FP64 : SGPU_FP32; }
-constexpr int LDS_LIMIT = 160 * 1024;
-constexpr int LDS_STATIC = 64; // the persistent Monte Carlo kernel's own LDS (its work item)
 constexpr double TUNE_MARGIN = 0.03; // a tuned plan must beat the default by this fraction
 // the speculative-chain kernel's own LDS (its request and result exchange)
 template<typename S>
@@ -647,8 +633,8 @@ TablePtrs<T> table_ptrs(const sgpu_ctx* c)
 	t.qsmooth = (sizeof(T) == 8 ? c->tab.qsmooth64 : c->tab.qsmooth32).template as<T>();
 	t.qfast = c->tab.qfast.as<double>();
 	t.n = c->tab.n;
-	t.factor = c->tab.factor;
-	t.cutoff_sqr = c->tab.cutoff_sqr;
+	t.factor_t = T(c->tab.factor);
+	t.cutoff_t = T(c->tab.cutoff_sqr);
 	t.kind = c->tab.kind;
 	t.spl = c->tab.spl.as<double>();
 	t.spl_cut = c->tab.spl_cut.as<double>();
@@ -668,13 +654,13 @@ GridPtrs<T> grid_ptrs(const Grid& g, double slope)
 	for (int d = 0; d < 3; d++)
 	{
 		p.dim[d] = g.dim[d];
-		p.init[d] = g.init[d];
-		p.factor[d] = g.factor[d];
-		p.factor_inv[d] = g.factor_inv[d];
-		p.dim_fl_minus_1[d] = g.dim_fl_minus_1[d];
+		p.init[d] = T(g.init[d]);
+		p.factor[d] = T(g.factor[d]);
+		p.factor_inv[d] = T(g.factor_inv[d]);
+		p.dim_fl_minus_1[d] = T(g.dim_fl_minus_1[d]);
 	}
 	p.ncells = (g.dim[0] - 1) * (g.dim[1] - 1) * (g.dim[2] - 1);
-	p.slope = slope;
+	p.slope = T(slope);
 	return p;
 }
 
@@ -706,10 +692,10 @@ void attach_user_grid(const sgpu_ctx* c, EvalCtx<T>& ec)
 	for (int d = 0; d < 3; d++)
 	{
 		p.dim[d] = c->ug.dim[d];
-		p.init[d] = c->ug.init[d];
-		p.factor[d] = c->ug.factor[d];
-		p.factor_inv[d] = c->ug.finv[d];
-		p.dim_fl_minus_1[d] = c->ug.dm1[d];
+		p.init[d] = T(c->ug.init[d]);
+		p.factor[d] = T(c->ug.factor[d]);
+		p.factor_inv[d] = T(c->ug.finv[d]);
+		p.dim_fl_minus_1[d] = T(c->ug.dm1[d]);
 	}
 	p.ncells = (p.dim[0] - 1) * (p.dim[1] - 1) * (p.dim[2] - 1);
 	p.slope = 0;
@@ -999,7 +985,9 @@ sgpu_status sgpu_mc_capacity(sgpu_ctx* c, int precision, int* chains)
 		                   : precision == SGPU_MIXED ? mc_blocks_per_cu<float, double>(1, 0)
 		                                             : mc_blocks_per_cu<float, float>(1, 0);
 		require(per_cu > 0, "occupancy query failed");
-		*chains = per_cu * p.multiProcessorCount;
+		// at most two per SIMD: the automatic chain split, and so the result
+		// of a --fast search, is defined by this number
+		*chains = std::min(per_cu, 8) * p.multiProcessorCount;
 	});
 }
 
@@ -1306,7 +1294,8 @@ sgpu_status sgpu_upload_models(sgpu_ctx* c, const sgpu_flat_model* models, int n
 		b->n = n;
 		pack_batch(models, n, b->h);
 		b->h.plan.bytes = plan_bytes(b->h.plan, precision, 1);
-		require(plan_bytes(b->h.plan, SGPU_FP64, 1) <= LDS_LIMIT && b->h.plan.bytes <= LDS_LIMIT,
+		require(limit_bytes(b->h.plan, b->h.limit, SGPU_FP64) <= LDS_LIMIT &&
+						limit_bytes(b->h.plan, b->h.limit, precision) <= LDS_LIMIT,
 				"model too large for one workgroup's LDS");
 		upload_batch(*b, c->stream);
 		if (precision != SGPU_FP64)
@@ -1489,19 +1478,35 @@ __global__ void early_stop_kernel(int nmodels, const int* mstart, const int* mch
 	}
 }
 
-// the occupancy rule of a size class: chains per workgroup for the most
-// resident waves per CU (registers and LDS, from the runtime's occupancy
-// calculator), then the larger workgroup; 0 when nothing fits
+// the default form: the persistent grid unless its kernel spills where the
+// one-shot kernel does not; SGPU_QUEUE=0 / 1 forces either
 template<typename T, typename S>
-int occupancy_waves(const WavePlan& plan, int precision, int variant, int maxper, int* resident)
+bool persist_default(int variant)
+{
+	const char* qenv = std::getenv("SGPU_QUEUE");
+	return qenv ? std::atoi(qenv) != 0 : mc_private_bytes<T, S>(variant, true) <= mc_private_bytes<T, S>(variant, false);
+}
+
+// the occupancy rule of a size class: chains per workgroup for the most
+// resident chains per CU (registers and LDS, from the runtime's occupancy
+// calculator, less the waves that a ligand's last workgroup leaves empty: 8
+// chains in workgroups of 6 fill 8 of 12), then the larger workgroup, and no
+// larger than `share`, an even share of the launch's chains per CU: larger
+// ones leave CUs empty while the chains of one CU wait for each other; 0 when
+// nothing fits
+template<typename T, typename S>
+int occupancy_waves(const WavePlan& plan, int precision, int variant, bool persist, int maxper, int share,
+		int* resident)
 {
 	int waves = 0, best = 0;
-	for (int w = 1; w <= std::min(MAX_CHAINS_PER_GROUP, maxper); w++)
+	for (int w = 1; w <= std::min({MAX_CHAINS_PER_GROUP, maxper, share}); w++)
 	{
 		const int bytes = plan_bytes(plan, precision, w);
 		if (bytes + LDS_STATIC > LDS_LIMIT)
 			break;
-		const int r = w * mc_blocks_per_cu<T, S>(w, size_t(bytes), variant);
+		const int per_cu = mc_blocks_per_cu<T, S>(w, size_t(bytes), variant, persist, false, plan.pair_lds);
+		const int groups = (maxper + w - 1) / w;
+		const int r = w * per_cu * maxper / (groups * w);
 		if (r >= best && r > 0)
 		{
 			best = r;
@@ -1511,15 +1516,6 @@ int occupancy_waves(const WavePlan& plan, int precision, int variant, int maxper
 	if (resident)
 		*resident = best;
 	return waves;
-}
-
-// the default form: the persistent grid unless its kernel spills where the
-// one-shot kernel does not; SGPU_QUEUE=0 / 1 forces either
-template<typename T, typename S>
-bool persist_default(int variant)
-{
-	const char* qenv = std::getenv("SGPU_QUEUE");
-	return qenv ? std::atoi(qenv) != 0 : mc_private_bytes<T, S>(variant, true) <= mc_private_bytes<T, S>(variant, false);
 }
 
 template<typename T, typename S>
@@ -1604,7 +1600,7 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 					const WavePlan pl = plan_for(b.h, k.models);
 					const int bytes = plan_bytes(pl, b.precision, w);
 					const int per_cu = bytes + spec_static_bytes<S>() <= LDS_LIMIT
-							? mc_blocks_per_cu<T, S>(w, size_t(bytes), variant, false, true)
+							? mc_blocks_per_cu<T, S>(w, size_t(bytes), variant, false, true, pl.pair_lds)
 							: 0;
 					slots = std::min(slots, per_cu * w * prop.multiProcessorCount);
 				}
@@ -1670,6 +1666,8 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 		scal[0] = 0;
 		scal[1] = Real_host_max<S>();
 	}
+	const bool pdef = persist_default<T, S>(variant);
+	const int share = std::max(1, (n + prop.multiProcessorCount - 1) / prop.multiProcessorCount);
 	std::vector<int> block_model, slot_chain;
 	for (Cls& k : cls)
 	{
@@ -1680,7 +1678,7 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 		for (int mi : k.models)
 			maxper = std::max(maxper, int(by_model[mi].size()));
 		// chains per workgroup by the occupancy rule
-		k.waves = occupancy_waves<T, S>(k.plan, b.precision, variant, maxper, &k.resident);
+		k.waves = occupancy_waves<T, S>(k.plan, b.precision, variant, pdef, maxper, share, &k.resident);
 		require(k.waves > 0, "chain state exceeds LDS");
 		// a probe's override, else the tuned plan of this class, where it fits
 		const int ki = int(&k - cls);
@@ -1699,12 +1697,12 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 			k.waves = spec;
 			k.spec = true;
 			k.resident = spec * mc_blocks_per_cu<T, S>(spec, size_t(plan_bytes(k.plan, b.precision, spec)), variant,
-					false, true);
+					false, true, k.plan.pair_lds);
 		}
 		else if (cp && cp->waves >= 1 && cp->waves <= std::min(MAX_CHAINS_PER_GROUP, maxper) &&
 				plan_bytes(k.plan, b.precision, cp->waves) + LDS_STATIC <= LDS_LIMIT &&
 				mc_blocks_per_cu<T, S>(cp->waves, size_t(plan_bytes(k.plan, b.precision, cp->waves)), variant,
-						cp->persist) > 0)
+						cp->persist, false, k.plan.pair_lds) > 0)
 		{
 			k.waves = cp->waves;
 			k.persist = cp->persist;
@@ -1794,7 +1792,6 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 	// the default form unless a tuned plan says otherwise
 	// SGPU_PERSIST_GRID caps a persistent grid's workgroups (each then runs
 	// more items)
-	const bool pdef = persist_default<T, S>(variant);
 	const char* genv = std::getenv("SGPU_PERSIST_GRID");
 	const int grid_cap = genv ? std::max(1, std::atoi(genv)) : std::numeric_limits<int>::max();
 	for (Cls& k : cls)
@@ -1803,7 +1800,7 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 			if (!k.tuned)
 				k.persist = pdef && !k.spec;
 			const int per_cu = mc_blocks_per_cu<T, S>(k.waves, size_t(plan_bytes(k.plan, b.precision, k.waves)),
-					variant, k.persist, k.spec);
+					variant, k.persist, k.spec, k.plan.pair_lds);
 			k.grid = k.persist ? std::max(1, std::min({int(k.blks.size()), per_cu * prop.multiProcessorCount, grid_cap}))
 			                   : int(k.blks.size());
 		}
@@ -2003,6 +2000,8 @@ void run_tune(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, c
 		members[mc_class(b.h.hdr[ch->model[i]])].push_back(i);
 		hmax = std::max(hmax, b.h.hdr[ch->model[i]].nheavy);
 	}
+	hipDeviceProp_t prop;
+	hip_check(hipGetDeviceProperties(&prop, c->device), "hipGetDeviceProperties");
 	*rep = sgpu_mc_tune_report{};
 	sgpu_mc_params probe = *p;
 	probe.early_stop_checkpoints = 0;
@@ -2045,7 +2044,7 @@ void run_tune(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, c
 		for (int w = std::min({target, MAX_CHAINS_PER_GROUP, info[k].maxper}); w >= 1; w--)
 		{
 			const int bytes = plan_bytes(info[k].plan, b.precision, w);
-			if (bytes + LDS_STATIC <= LDS_LIMIT && mc_blocks_per_cu<T, S>(w, size_t(bytes), variant, pers) > 0)
+			if (bytes + LDS_STATIC <= LDS_LIMIT && mc_blocks_per_cu<T, S>(w, size_t(bytes), variant, pers, false, info[k].plan.pair_lds) > 0)
 				return w;
 		}
 		return 0;
@@ -2065,7 +2064,9 @@ void run_tune(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, c
 		Joint d{};
 		for (int k = 0; k < sgpu_ctx::NCLASS; k++)
 			if (!members[k].empty())
-				d.plan[k] = {occupancy_waves<T, S>(info[k].plan, b.precision, variant, info[k].maxper, nullptr),
+				d.plan[k] = {occupancy_waves<T, S>(info[k].plan, b.precision, variant, persist_default<T, S>(variant),
+								info[k].maxper,
+								std::max(1, (ch->nchains + prop.multiProcessorCount - 1) / prop.multiProcessorCount), nullptr),
 						persist_default<T, S>(variant)};
 		cands.push_back(d);
 	}

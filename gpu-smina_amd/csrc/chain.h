@@ -120,8 +120,9 @@ __device__ inline S conf_increment(const MV<T>& m, const SearchMem<S>& W, S alph
 	const int k = lane_id();
 	if (k >= m.h.conf_size)
 		return S(0);
-	const int kind = m.ckind[k];
-	const int gi = m.cchg[k];
+	const int cm = m.cmap[k];
+	const int kind = map_kind(cm);
+	const int gi = map_index(cm);
 	const S x = W.xstage[k];
 	if (kind == CK_POSITION)
 	{
@@ -149,8 +150,9 @@ __device__ inline S conf_value(const MV<T>& m, const SearchMem<S>& W)
 	const int i = lane_id();
 	if (i >= m.h.change_size)
 		return S(0);
-	const int kind = m.gkind[i];
-	const int ci = m.gconf[i];
+	const int gm = m.gmap[i];
+	const int kind = map_kind(gm);
+	const int ci = map_index(gm);
 	if (kind == GK_POSITION || kind == GK_TORSION)
 		return W.xstage[ci];
 	const Q4<S> q = {W.xstage[ci], W.xstage[ci + 1], W.xstage[ci + 2], W.xstage[ci + 3]};
@@ -319,7 +321,7 @@ struct SpecLink
 // point, then the line search's trials; a finished line search runs the
 // BFGS step body and starts the next line search.  The order of every
 // evaluation and every arithmetic operation is the CPU's.
-template<typename T, typename S, int BK, bool VIS = false, bool SPL = true, bool SPEC = false>
+template<typename T, typename S, int BK, bool VIS = false, bool SPL = true, bool SPEC = false, bool PS = true>
 struct Searcher
 {
 	const MV<T>& m;
@@ -403,7 +405,7 @@ struct Searcher
 		{
 			++evals;
 			T ge_t;
-			const S fe = S(eval_deriv<T, BK, SPL>(m, ec, W, pbuf, T(xe), ge_t));
+			const S fe = S(eval_deriv<T, BK, SPL, PS>(m, ec, W, pbuf, T(xe), ge_t));
 			const S ge = S(ge_t);
 			helper_last = false;
 			bool begin = false;
@@ -630,7 +632,7 @@ struct Searcher
 // the evaluation at the top of Searcher::bfgs do, and leave its energy, conf
 // and gradient for wave 0.  Two workgroup barriers per round (A, B), as wave
 // 0 takes them.
-template<typename T, typename S, bool SPL>
+template<typename T, typename S, bool SPL, bool PS>
 __device__ inline void spec_helper(const MV<T>& m, const EvalCtx<T>& ec, WaveMem<T>& W, SearchMem<S>& SM,
 		const SpecLink<S>& L, int rank, T* pbuf)
 {
@@ -653,7 +655,7 @@ __device__ inline void spec_helper(const MV<T>& m, const EvalCtx<T>& ec, WaveMem
 		const S xe = conf_increment(m, SM, alpha);
 		lsync();
 		T g;
-		const S f = S(eval_deriv<T, BK_MAPS, SPL>(m, ev, W, pbuf, T(xe), g));
+		const S f = S(eval_deriv<T, BK_MAPS, SPL, PS>(m, ev, W, pbuf, T(xe), g));
 		S* r = L.res + rank * SPEC_RS;
 		if (lane == 0)
 			r[0] = f;
@@ -818,16 +820,15 @@ struct McParams
 template<typename T>
 __device__ inline double gyration_radius(const MV<T>& m, const WaveMem<T>& W, int tree)
 {
-	const int root = m.troot[tree];
-	const V3<T> o = ld3(W.fo + 3 * root);
+	const V3<T> o = frame_origin(W, m.tr(tree, TR_ROOT));
 	T acc = 0;
 	unsigned counter = 0;
 	if constexpr (Real<T>::ordered)
 	{
-		for (int i = m.tab_[tree]; i < m.tae[tree]; i++)
-			if (!is_hydrogen_type(m.type[i]))
+		for (int i = m.tr(tree, TR_AB); i < m.tr(tree, TR_AE); i++)
+			if (atom_heavy(m.am[i].x))
 			{
-				const V3<T> x = ld3(W.coords + 3 * i);
+				const V3<T> x = ld_atom(W.coords, i);
 				acc += sqr(x.x - o.x) + sqr(x.y - o.y) + sqr(x.z - o.z);
 				++counter;
 			}
@@ -835,10 +836,10 @@ __device__ inline double gyration_radius(const MV<T>& m, const WaveMem<T>& W, in
 	else
 	{
 		T part = 0, cnt = 0;
-		for (int i = m.tab_[tree] + lane_id(); i < m.tae[tree]; i += WAVE)
-			if (!is_hydrogen_type(m.type[i]))
+		for (int i = m.tr(tree, TR_AB) + lane_id(); i < m.tr(tree, TR_AE); i += WAVE)
+			if (atom_heavy(m.am[i].x))
 			{
-				const V3<T> x = ld3(W.coords + 3 * i);
+				const V3<T> x = ld_atom(W.coords, i);
 				part += sqr(x.x - o.x) + sqr(x.y - o.y) + sqr(x.z - o.z);
 				cnt += 1;
 			}
@@ -856,15 +857,15 @@ __device__ inline S mutate(const MV<T>& m, const WaveMem<T>& W, S x, double ampl
 	const int lane = lane_id();
 	int count = 0;
 	for (int t = 0; t < m.h.ntrees; t++)
-		count += m.tlig[t] ? 2 + m.tntors[t] : m.tntors[t];
+		count += m.tr(t, TR_LIG) ? 2 + m.tr(t, TR_NTORS) : m.tr(t, TR_NTORS);
 	if (count == 0)
 		return x;
 	int which = random_int(0, count - 1, g);
 	for (int t = 0; t < m.h.ntrees; t++)
 	{
-		if (!m.tlig[t])
+		if (!m.tr(t, TR_LIG))
 			continue;
-		const int cc = m.tconf[t];
+		const int cc = m.tr(t, TR_CONF);
 		if (which == 0)
 		{
 			const V3<double> s = random_inside_sphere(g);
@@ -900,27 +901,27 @@ __device__ inline S mutate(const MV<T>& m, const WaveMem<T>& W, S x, double ampl
 			return x;
 		}
 		--which;
-		if (which < m.tntors[t])
+		if (which < m.tr(t, TR_NTORS))
 		{
 			const double v = random_fl(-3.1415926535897931, 3.1415926535897931, g);
 			if (lane == cc + 7 + which)
 				x = S(v);
 			return x;
 		}
-		which -= m.tntors[t];
+		which -= m.tr(t, TR_NTORS);
 	}
 	for (int t = 0; t < m.h.ntrees; t++)
 	{
-		if (m.tlig[t])
+		if (m.tr(t, TR_LIG))
 			continue;
-		if (which < m.tntors[t])
+		if (which < m.tr(t, TR_NTORS))
 		{
 			const double v = random_fl(-3.1415926535897931, 3.1415926535897931, g);
-			if (lane == m.tconf[t] + which)
+			if (lane == m.tr(t, TR_CONF) + which)
 				x = S(v);
 			return x;
 		}
-		which -= m.tntors[t];
+		which -= m.tr(t, TR_NTORS);
 	}
 	return x;
 }
@@ -952,7 +953,7 @@ __device__ inline void add_to_output(const MV<T>& m, const WaveMem<T>& W, ChainS
 		T acc = 0;
 		for (int h = 0; h < H; h++)
 		{
-			const V3<T> a = ld3(W.coords + 3 * m.heavy[h]);
+			const V3<T> a = ld_atom(W.coords, m.heavy[h]);
 			acc += sqr(a.x - oc[3 * h]) + sqr(a.y - oc[3 * h + 1]) + sqr(a.z - oc[3 * h + 2]);
 		}
 		rmsd = H > 0 ? Real<T>::sqrt(acc / T(H)) : T(0);
@@ -992,7 +993,7 @@ __device__ inline void add_to_output(const MV<T>& m, const WaveMem<T>& W, ChainS
 			s.out_conf[size_t(slot) * L.conf_stride + lane] = x;
 		for (int h = lane; h < H; h += WAVE)
 		{
-			const V3<T> a = ld3(W.coords + 3 * m.heavy[h]);
+			const V3<T> a = ld_atom(W.coords, m.heavy[h]);
 			st3(s.out_coords + size_t(slot) * L.coord_stride + 3 * h, a);
 		}
 		if (lane == 0)
@@ -1025,9 +1026,9 @@ __device__ inline bool within_box(const MV<T>& m, const WaveMem<T>& W, const Rec
 	bool ok = true;
 	for (int i = lane_id(); i < m.h.natoms; i += WAVE)
 	{
-		if (is_hydrogen_type(m.type[i]))
+		if (!atom_heavy(m.am[i].x))
 			continue;
-		const V3<T> x = ld3(W.coords + 3 * i);
+		const V3<T> x = ld_atom(W.coords, i);
 		const T c[3] = {x.x, x.y, x.z};
 		for (int j = 0; j < 3; j++)
 			if (r.enabled[j])

@@ -21,6 +21,7 @@ struct GridSample
 	T s[3];     // position inside the cell
 	T miss[3];  // distance outside the box along each axis (grid units)
 	int region[3];
+	bool inside; // uniform: every lane's location is inside the box
 };
 
 // the corners from `cells` (a map set laid out as g.cells: the receptor
@@ -29,37 +30,39 @@ template<typename T>
 __device__ inline GridSample<T> grid_fetch(const GridPtrs<T>& g, const T* cells, int slot, V3<T> loc)
 {
 	GridSample<T> r;
-	r.s[0] = (loc.x - T(g.init[0])) * T(g.factor[0]);
-	r.s[1] = (loc.y - T(g.init[1])) * T(g.factor[1]);
-	r.s[2] = (loc.z - T(g.init[2])) * T(g.factor[2]);
+	r.s[0] = (loc.x - g.init[0]) * g.factor[0];
+	r.s[1] = (loc.y - g.init[1]) * g.factor[1];
+	r.s[2] = (loc.z - g.init[2]) * g.factor[2];
 	int a[3];
+	bool out = false;
 	for (int i = 0; i < 3; i++)
+		out = out || !(r.s[i] >= 0 && r.s[i] < g.dim_fl_minus_1[i]);
+	r.inside = wave_all(!out);
+	if (r.inside)
 	{
-		const T dm1 = T(g.dim_fl_minus_1[i]);
-		r.miss[i] = 0;
-		if (r.s[i] < 0)
+		// every active lane's atom is inside the box (nearly every call of a
+		// search): no clamping, no penalty
+		for (int i = 0; i < 3; i++)
 		{
-			r.miss[i] = -r.s[i];
-			r.region[i] = -1;
-			a[i] = 0;
-			r.s[i] = 0;
-		}
-		else if (r.s[i] >= dm1)
-		{
-			r.miss[i] = r.s[i] - dm1;
-			r.region[i] = 1;
-			a[i] = g.dim[i] - 2;
-			r.s[i] = 1;
-		}
-		else
-		{
-			r.region[i] = 0;
 			a[i] = int(r.s[i]);
 			r.s[i] -= T(a[i]);
+			r.miss[i] = 0;
+			r.region[i] = 0;
 		}
-		// in range for every finite location; keeps a NaN location's gather in bounds
-		a[i] = a[i] < 0 ? 0 : (a[i] > g.dim[i] - 2 ? g.dim[i] - 2 : a[i]);
 	}
+	else
+		for (int i = 0; i < 3; i++)
+		{
+			const T dm1 = g.dim_fl_minus_1[i], s = r.s[i];
+			const bool below = s < 0, above = s >= dm1;
+			const int cell = int(s);
+			r.miss[i] = below ? -s : above ? s - dm1 : T(0);
+			r.region[i] = below ? -1 : above ? 1 : 0;
+			a[i] = below ? 0 : above ? g.dim[i] - 2 : cell;
+			r.s[i] = below ? T(0) : above ? T(1) : s - T(cell);
+			// in range for every finite location; keeps a NaN location's gather in bounds
+			a[i] = a[i] < 0 ? 0 : (a[i] > g.dim[i] - 2 ? g.dim[i] - 2 : a[i]);
+		}
 	const size_t cell = size_t(a[0]) + size_t(g.dim[0] - 1) * (size_t(a[1]) + size_t(g.dim[1] - 1) * a[2]);
 	const T* c = cells + (size_t(slot) * g.ncells + cell) * 8;
 	for (int k = 0; k < 8; k++)
@@ -76,8 +79,6 @@ __device__ inline GridSample<T> grid_fetch(const GridPtrs<T>& g, int slot, V3<T>
 template<typename T>
 __device__ inline T grid_finish(const GridPtrs<T>& g, const GridSample<T>& r, T v, T slope, V3<T>& deriv)
 {
-	const T penalty = slope * (r.miss[0] * T(g.factor_inv[0]) + r.miss[1] * T(g.factor_inv[1]) +
-			r.miss[2] * T(g.factor_inv[2]));
 	const T f000 = r.c[0], f100 = r.c[1], f010 = r.c[2], f110 = r.c[3];
 	const T f001 = r.c[4], f101 = r.c[5], f011 = r.c[6], f111 = r.c[7];
 	const T x = r.s[0], y = r.s[1], z = r.s[2];
@@ -94,11 +95,19 @@ __device__ inline T grid_finish(const GridPtrs<T>& g, const GridSample<T>& r, T 
 	V3<T> grad = v3(x_g, y_g, z_g);
 	curl(f, grad, v);
 	const T gr[3] = {grad.x, grad.y, grad.z};
+	if (r.inside)
+	{
+		// no penalty, and slope x 0 adds nothing to the derivative
+		deriv = v3(g.factor[0] * gr[0], g.factor[1] * gr[1], g.factor[2] * gr[2]);
+		return f;
+	}
+	const T penalty = slope * (r.miss[0] * g.factor_inv[0] + r.miss[1] * g.factor_inv[1] +
+			r.miss[2] * g.factor_inv[2]);
 	T d[3];
 	for (int i = 0; i < 3; i++)
 	{
 		const T ge = r.region[i] == 0 ? gr[i] : T(0);
-		d[i] = T(g.factor[i]) * ge + slope * T(r.region[i]);
+		d[i] = g.factor[i] * ge + slope * T(r.region[i]);
 	}
 	deriv = v3(d[0], d[1], d[2]);
 	return f + penalty;
@@ -107,7 +116,7 @@ __device__ inline T grid_finish(const GridPtrs<T>& g, const GridSample<T>& r, T 
 template<typename T>
 __device__ inline T grid_finish(const GridPtrs<T>& g, const GridSample<T>& r, T v, V3<T>& deriv)
 {
-	return grid_finish(g, r, v, T(g.slope), deriv);
+	return grid_finish(g, r, v, g.slope, deriv);
 }
 
 template<typename T>
@@ -134,8 +143,8 @@ template<typename T>
 __device__ inline T grid_value(const GridPtrs<T>& g, V3<T> loc, T v, T slope)
 {
 	const GridSample<T> r = grid_fetch(g, 0, loc);
-	const T penalty = slope * (r.miss[0] * T(g.factor_inv[0]) + r.miss[1] * T(g.factor_inv[1]) +
-			r.miss[2] * T(g.factor_inv[2]));
+	const T penalty = slope * (r.miss[0] * g.factor_inv[0] + r.miss[1] * g.factor_inv[1] +
+			r.miss[2] * g.factor_inv[2]);
 	const T f000 = r.c[0], f100 = r.c[1], f010 = r.c[2], f110 = r.c[3];
 	const T f001 = r.c[4], f101 = r.c[5], f011 = r.c[6], f111 = r.c[7];
 	const T x = r.s[0], y = r.s[1], z = r.s[2];

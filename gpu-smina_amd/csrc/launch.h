@@ -36,8 +36,9 @@ hipError_t launch_mc(const BatchPtrs<T>& B, const EvalCtx<T>& ec, const WavePlan
 template<typename T, typename S>
 // variant: 0 smina's search, 1 with QuickVina 2's history, 2 with the
 // spline or charge-dependent tables (and the history); spec: the
-// speculative-chain kernel (waves = its width)
-int mc_blocks_per_cu(int waves, size_t lds, int variant = 0, bool persist = false, bool spec = false);
+// speculative-chain kernel (waves = its width); ps: the plan holds its pairs
+// in LDS
+int mc_blocks_per_cu(int waves, size_t lds, int variant = 0, bool persist = false, bool spec = false, bool ps = true);
 // per-lane private (scratch) bytes of a Monte Carlo kernel form: register
 // spills, which the persistent form must not add
 template<typename T, typename S>

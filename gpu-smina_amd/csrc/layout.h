@@ -9,20 +9,23 @@
  * same ligand) reads the model from LDS only.  ModelHdr holds the counts
  * and each array's offset inside the blobs.
  *
- * int blob:  atom type (movable then fixed atoms), atom frame, per-atom
- *            neighbour lists (start, packed codes), frames (parent, kind,
- *            atom range, conf / change index, children), tree levels, heavy
- *            atoms, trees, conf / change maps;
- * real blob: initial coordinates (movable then fixed), local coordinates,
- *            frame origins and axes (segment: relative to the parent),
- *            partial charges (movable then fixed).
+ * int blob:  movable atoms' records (two words: frame, type, heavy flag and
+ *            map slot; the range of the neighbour list), atom types (movable
+ *            then fixed), neighbour codes, pair records, frame records, paths
+ *            and children, heavy atoms, trees, conf / change maps;
+ * real blob: initial coordinates (movable then fixed, 3 reals each), local
+ *            coordinates, frame origins and axes (4 reals each; segment:
+ *            relative to the parent), partial charges (movable then fixed).
+ * Packed records keep the addresses a wave holds few: with an array for each
+ * field the search kernels held some 100 uniform values and moved 130 to 300
+ * of them through vector lanes.
  *
- * A neighbour code is one 32-bit word: the partner atom (bits 0-7), the
- * type-pair table index (8-16), "this atom is the pair's b" (17), "the pair
- * is an other pair" (18) and the pair index (19-31), so the pair loop reads
- * one LDS word per neighbour.  The pair-parallel loop of the FP32 search
- * reads the pairs themselves, two words each (coordinate offsets of a and
- * b; table index and "other pair").
+ * A neighbour code is one word: the partner atom (bits 0-15) and the pair's
+ * slot, its index plus one (16-31).  Each atom's list is padded to a multiple
+ * of 4 codes with entries of slot 0 (the atom itself, no force), so that a
+ * lane reads 4 codes at once and needs no check for the end of its list.  A
+ * pair record is one word: atoms a (0-7) and b (8-15), the table index
+ * (16-24).
  *
  * Receptor maps are stored per ligand type as corner-packed cells: for each
  * grid cell (x fastest), its 8 corner values in the order f000 f100 f010
@@ -63,37 +66,86 @@ enum ChangeKind
 	GK_TORSION = 4
 };
 
-__host__ __device__ inline int code_partner(int c) { return c & 255; }
-__host__ __device__ inline int code_tri(int c) { return (c >> 8) & 511; }
-__host__ __device__ inline bool code_is_b(int c) { return (c >> 17) & 1; }
-__host__ __device__ inline bool code_other(int c) { return (c >> 18) & 1; }
-__host__ __device__ inline int code_pair(int c) { return int(unsigned(c) >> 19); }
-__host__ __device__ inline int make_code(int partner, int tri, bool is_b, bool other, int pair)
-{
-	return int(unsigned(partner) | (unsigned(tri) << 8) | (unsigned(is_b) << 17) | (unsigned(other) << 18) |
-			(unsigned(pair) << 19));
-}
+constexpr int NBR_BATCH = 4; // codes a neighbour list is padded to
+__host__ __device__ inline int make_code(int partner, int slot) { return int(unsigned(partner) | (unsigned(slot) << 16)); }
+__host__ __device__ inline int code_partner(int c) { return c & 0xffff; }
+__host__ __device__ inline int code_slot(int c) { return int(unsigned(c) >> 16); }
 
-// pair record of the pair-parallel loop: two words, the coordinate offsets
-// 3a (bits 0-15) and 3b (16-31), then the table index (0-15) and "other
-// pair" (16)
-__host__ __device__ inline int prec_xa(int w0) { return w0 & 0xffff; }
-__host__ __device__ inline int prec_xb(int w0) { return int(unsigned(w0) >> 16); }
-__host__ __device__ inline int prec_tri(int w1) { return w1 & 0xffff; }
-__host__ __device__ inline bool prec_other(int w1) { return (w1 >> 16) & 1; }
+// pair record: atoms a and b, table index
+__host__ __device__ inline int make_prec(int a, int b, int tri) { return a | (b << 8) | (tri << 16); }
+__host__ __device__ inline int prec_a(int w) { return w & 255; }
+__host__ __device__ inline int prec_b(int w) { return (w >> 8) & 255; }
+__host__ __device__ inline int prec_tri(int w) { return w >> 16; }
+
+// movable atom's record: word 0 frame (0-7), type (8-15), map slot (16-23),
+// heavy (24); word 1 first neighbour code (0-15) and the one past the last
+// (16-31)
+__host__ __device__ inline int make_atom(int frame, int type, bool heavy) { return frame | (type << 8) | (int(heavy) << 24); }
+__host__ __device__ inline int atom_frame(int w) { return w & 255; }
+__host__ __device__ inline int atom_type_of(int w) { return (w >> 8) & 255; }
+__host__ __device__ inline int atom_slot(int w) { return (w >> 16) & 255; }
+__host__ __device__ inline bool atom_heavy(int w) { return (w >> 24) & 1; }
+__host__ __device__ inline int atom_with_slot(int w, int slot) { return (w & ~(255 << 16)) | ((slot & 255) << 16); }
+__host__ __device__ inline int atom_nbr_begin(int w) { return w & 0xffff; }
+__host__ __device__ inline int atom_nbr_end(int w) { return int(unsigned(w) >> 16); }
+
+// frame's record: word 0 kind (0-7), conf index (8-15), change index
+// (16-23), depth in its tree (24-31); word 1 atom range begin (0-7), end of
+// the subtree's atoms (8-15), end (16-23), parent (24-31, 255: none)
+__host__ __device__ inline int make_frame0(int kind, int conf, int change, int depth)
+{
+	return kind | (conf << 8) | (change << 16) | (depth << 24);
+}
+__host__ __device__ inline int make_frame1(int begin, int send, int end, int parent)
+{
+	return int(unsigned(begin) | (unsigned(send) << 8) | (unsigned(end) << 16) | (unsigned(parent) << 24));
+}
+__host__ __device__ inline int frame_kind(int w) { return w & 255; }
+__host__ __device__ inline int frame_conf(int w) { return (w >> 8) & 255; }
+__host__ __device__ inline int frame_change(int w) { return (w >> 16) & 255; }
+__host__ __device__ inline int frame_depth(int w) { return int(unsigned(w) >> 24); }
+__host__ __device__ inline int frame_begin(int w) { return w & 255; }
+__host__ __device__ inline int frame_send(int w) { return (w >> 8) & 255; }
+__host__ __device__ inline int frame_end(int w) { return (w >> 16) & 255; }
+__host__ __device__ inline int frame_parent(int w) { return int(unsigned(w) >> 24); }
+// a frame's children: first entry of the children list and their number
+__host__ __device__ inline int make_child(int start, int count) { return start | (count << 8); }
+__host__ __device__ inline int child_start(int w) { return w & 255; }
+__host__ __device__ inline int child_count(int w) { return w >> 8; }
+
+// per tree: root frame, conf and change index of the root, ligand flag,
+// torsions, atom range, ligand-internal pair range
+enum TreeField
+{
+	TR_ROOT = 0,
+	TR_CONF,
+	TR_CHANGE,
+	TR_LIG,
+	TR_NTORS,
+	TR_AB,
+	TR_AE,
+	TR_PB,
+	TR_PE,
+	TR_FIELDS
+};
+
+// conf / change map entry: the element's kind, and the other space's index
+// (orientation: its first)
+__host__ __device__ inline int make_map(int kind, int index) { return kind | (index << 8); }
+__host__ __device__ inline int map_kind(int w) { return w & 255; }
+__host__ __device__ inline int map_index(int w) { return w >> 8; }
 
 struct ModelHdr
 {
 	int natoms, ninflex, nframes, ntrees, nligands, npairs, nother;
 	int conf_size, change_size, nheavy, nlevels, num_tors;
 	int path_ok; // every root-to-frame path has at most MAX_PATH frames
+	int ncodes;
+	int one_ligand; // one ligand whose pairs are all those after the other pairs
 	int iblob_off, iblob_len; // in the batch int blob
 	int tblob_off, tblob_len; // in the batch real blob
-	int pair_off;             // pair arrays (a, b, table index), global
-	// offsets inside the int blob
-	int o_type, o_afr, o_nbr, o_code, o_prec, o_fparent, o_fkind, o_fbegin, o_fend, o_fconf, o_fchange, o_fsend, o_fdepth, o_fpath, o_cstart,
-			o_ccount, o_clist, o_lstart, o_lframes, o_heavy, o_troot, o_tconf, o_tchange, o_tlig, o_tntors,
-			o_tab, o_tae, o_tpb, o_tpe, o_maps;
+	// offsets inside the int blob (the movable atoms' records at 0)
+	int o_type, o_code, o_prec, o_fm, o_fpath, o_child, o_clist, o_heavy, o_tree, o_cmap, o_gmap;
 	// offsets inside the real blob
 	int o_xyz0, o_local, o_forig, o_faxis, o_charge;
 };
@@ -104,9 +156,6 @@ struct BatchPtrs
 	const ModelHdr* hdr;
 	const int* iblob;
 	const T* tblob;
-	const int* pair_a;
-	const int* pair_b;
-	const int* pair_tri;
 };
 
 // scoring tables on the device: smooth as (e, dor) pairs per point; fast
@@ -123,8 +172,8 @@ struct TablePtrs
 	const T* qsmooth;    // [378][n][3][2] (ncomp 4)
 	const double* qfast; // [378][n][3] (ncomp 4)
 	int n;
-	double factor;
-	double cutoff_sqr;
+	T factor_t;          // points per A^2 and the squared cutoff in the evaluation's precision
+	T cutoff_t;
 	// precalculate_splines (kind 1; FP64 direct evaluation only)
 	int kind;            // 0: linear tables, 1: splines
 	const double* spl;   // [378][nseg][5]: x, a, b, c, d
@@ -142,11 +191,11 @@ struct GridPtrs
 	const int* slot_of;  // [27] -> map slot or -1
 	int dim[3];          // points per axis
 	int ncells;          // (dim0-1)(dim1-1)(dim2-1)
-	double init[3];
-	double factor[3];
-	double factor_inv[3];
-	double dim_fl_minus_1[3];
-	double slope;
+	T init[3];
+	T factor[3];
+	T factor_inv[3];
+	T dim_fl_minus_1[3];
+	T slope;
 };
 
 // one entry of a cell's list of receptor atoms, in one 16-byte (FP32) or

@@ -19,7 +19,22 @@ namespace sgpu
 {
 
 __device__ inline int lane_id() { return int(threadIdx.x) & (WAVE - 1); }
-__device__ inline int wave_in_block() { return int(threadIdx.x) / WAVE; }
+// (uniform, and known to the compiler as such: addresses made from it are
+// scalar)
+__device__ inline int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ inline int wave_in_block() { return uniform(int(threadIdx.x) / WAVE); }
+
+// A uniform value in scalar registers of its own.  Values loaded together
+// (kernel arguments, the model header) arrive in groups of 16 registers that
+// the compiler spills and reloads whole: one use of one of them then costs 16
+// lane reads.
+template<typename X>
+__device__ __forceinline__ X own(X v)
+{
+	static_assert(sizeof(X) == 4 || sizeof(X) == 8, "a scalar");
+	asm("" : "+s"(v));
+	return v;
+}
 
 // Syncs inside one wavefront; waves never wait for each other.
 // lsync: LDS written by some lanes is read by others next.  A wavefront's
@@ -197,6 +212,12 @@ template<typename T> __device__ inline Q4<T> qmul(Q4<T> l, Q4<T> r)
 template<typename T> __device__ inline void normalize_angle(T& x)
 {
 	const T pi = T(3.1415926535897931);
+	if (wave_all(x >= -3 * pi && x <= 3 * pi))
+	{
+		// every active lane within one turn of the range: selects
+		x = x > pi ? x - 2 * pi : x < -pi ? x + 2 * pi : x;
+		return;
+	}
 	for (;;)
 	{
 		if (x > 3 * pi)
