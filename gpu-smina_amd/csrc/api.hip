@@ -17,6 +17,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <queue>
 #include <string>
 #include <vector>
 
@@ -1518,6 +1519,86 @@ int occupancy_waves(const WavePlan& plan, int precision, int variant, bool persi
 	return waves;
 }
 
+// the widths at which single chains of a launch speculate, and what the
+// helpers gain: a ligand's chains ran in 570 ms, 398 ms with one helper each
+// and 347 ms with three (67 atoms, 1,411 pairs), other ligands in 1,151, 746
+// and 584 ms (50 atoms); seven helpers gain no more
+constexpr int SPEC_WIDTHS = 2;
+constexpr int SPEC_WIDTH[SPEC_WIDTHS] = {2, 4};
+constexpr double SPEC_GAIN[SPEC_WIDTHS] = {1.45, 1.75};
+
+// a chain as the launch plan sees it: its cost, and the share of a CU (of its
+// LDS and wave slots) that it takes alone or with the helpers of each width
+// (0: does not fit)
+struct PlanChain
+{
+	double cost;
+	double share[1 + SPEC_WIDTHS];
+};
+
+// When the launch ends if the chains run at these width indices (0: no
+// helpers): the longest start first, each as soon as its share of `cus` CUs
+// is free.  A tenth of the device is left to workgroups that don't fill
+// their CU.
+double plan_end(const std::vector<PlanChain>& ch, const std::vector<int>& width, int cus)
+{
+	std::vector<std::pair<double, double>> items; // duration, share
+	for (size_t i = 0; i < ch.size(); i++)
+		items.push_back({width[i] ? ch[i].cost / SPEC_GAIN[width[i] - 1] : ch[i].cost, ch[i].share[width[i]]});
+	std::sort(items.begin(), items.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
+	std::priority_queue<std::pair<double, double>, std::vector<std::pair<double, double>>, std::greater<>> running;
+	double now = 0, end = 0, room = 0.9 * cus;
+	for (const auto& it : items)
+	{
+		while (room < it.second && !running.empty())
+		{
+			now = running.top().first;
+			room += running.top().second;
+			running.pop();
+		}
+		room -= it.second;
+		running.push({now + it.first, it.second});
+		end = std::max(end, now + it.first);
+	}
+	return end;
+}
+
+// The width index of every chain of a launch with more chains than can all
+// speculate.  Such a launch often lasts as long as its longest chains, so for
+// a range of ends, every chain that would run past the end takes the smallest
+// width that finishes it by then; the assignment whose launch ends soonest
+// (plan_end) is taken if it beats no speculation by 5%.  A launch whose chains
+// fill the device to the end gains nothing and keeps every chain alone.
+std::vector<int> critical_widths(const std::vector<PlanChain>& ch, int cus)
+{
+	std::vector<int> best(ch.size(), 0);
+	double longest = 0;
+	for (const PlanChain& c : ch)
+		longest = std::max(longest, c.cost);
+	// past this many chains no single one holds up the launch
+	if (longest <= 0 || ch.size() > 65536)
+		return best;
+	double best_end = 0.95 * plan_end(ch, best, cus);
+	for (double end = 0.95; end > 0.55; end -= 0.05)
+	{
+		std::vector<int> w(ch.size(), 0);
+		for (size_t i = 0; i < ch.size(); i++)
+			if (ch[i].cost > end * longest)
+			{
+				w[i] = ch[i].cost / SPEC_GAIN[0] <= end * longest ? 1 : 2;
+				while (w[i] > 0 && ch[i].share[w[i]] <= 0)
+					w[i]--;
+			}
+		const double t = plan_end(ch, w, cus);
+		if (t < best_end)
+		{
+			best_end = t;
+			best = w;
+		}
+	}
+	return best;
+}
+
 template<typename T, typename S>
 void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, const sgpu_chains* ch,
 		sgpu_chain_results* out)
@@ -1560,9 +1641,18 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 		int model;
 		std::vector<int> chains;
 	};
+	// the chains of one launch: a size class, or the longest chains at one
+	// speculation width
 	struct Cls
 	{
-		std::vector<int> models;
+		std::map<int, std::vector<int>> members; // model -> its chains
+		std::vector<int> models() const
+		{
+			std::vector<int> m;
+			for (auto& kv : members)
+				m.push_back(kv.first);
+			return m;
+		}
 		WavePlan plan;
 		int waves = 1;
 		int resident = 0; // waves per CU
@@ -1573,9 +1663,10 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 		std::vector<Blk> blks;
 		size_t block_off = 0, slot_off = 0;
 	};
-	Cls cls[sgpu_ctx::NCLASS];
+	constexpr int NGROUP = sgpu_ctx::NCLASS + SPEC_WIDTHS;
+	Cls cls[NGROUP];
 	for (auto& kv : by_model)
-		cls[class_of(kv.first)].models.push_back(kv.first);
+		cls[class_of(kv.first)].members.insert(kv);
 	hipDeviceProp_t prop;
 	hip_check(hipGetDeviceProperties(&prop, c->device), "hipGetDeviceProperties");
 	const int variant = (c->tab.kind == 1 || c->tab.ncomp == 4) ? 2 : p->visited ? 1 : 0;
@@ -1584,30 +1675,94 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 	// next trials of its fast line search), without QuickVina 2's history;
 	// the widest of 8, 4 and 2 whose n x width waves all fit at once.
 	// SGPU_SPEC=1 turns it off, 2..8 forces the width.
+	auto spec_per_cu = [&](const WavePlan& pl, int w) {
+		const int bytes = plan_bytes(pl, b.precision, w);
+		return bytes + spec_static_bytes<S>() <= LDS_LIMIT
+				? mc_blocks_per_cu<T, S>(w, size_t(bytes), variant, false, true, pl.pair_lds)
+				: 0;
+	};
 	int spec = 1;
-	if (!p->visited && !p->accurate_line_search)
-	{
-		const char* senv = std::getenv("SGPU_SPEC");
-		const int forced = senv ? std::atoi(senv) : 0;
+	bool hybrid = false; // some chains speculate
+	const char* senv = std::getenv("SGPU_SPEC");
+	const int forced = senv ? std::atoi(senv) : 0;
+	const bool may_speculate = !p->visited && !p->accurate_line_search;
+	if (may_speculate)
 		for (int w : {8, 4, 3, 2})
 		{
 			if (forced ? w != forced : w == 3)
 				continue;
 			int slots = std::numeric_limits<int>::max();
 			for (Cls& k : cls)
-				if (!k.models.empty())
-				{
-					const WavePlan pl = plan_for(b.h, k.models);
-					const int bytes = plan_bytes(pl, b.precision, w);
-					const int per_cu = bytes + spec_static_bytes<S>() <= LDS_LIMIT
-							? mc_blocks_per_cu<T, S>(w, size_t(bytes), variant, false, true, pl.pair_lds)
-							: 0;
-					slots = std::min(slots, per_cu * w * prop.multiProcessorCount);
-				}
+				if (!k.members.empty())
+					slots = std::min(slots, spec_per_cu(plan_for(b.h, k.models()), w) * w * prop.multiProcessorCount);
 			if (forced ? slots > 0 : int64_t(n) * w <= int64_t(slots))
 			{
 				spec = w;
 				break;
+			}
+		}
+	const bool pdef = persist_default<T, S>(variant);
+	const int share = std::max(1, (n + prop.multiProcessorCount - 1) / prop.multiProcessorCount);
+	// a chain's cost: its steps, the evaluations of a step (about as many per
+	// BFGS iteration for every model) and the time of one, 8.1 us + 5.8 ns a
+	// pair on a full device
+	auto cost_of = [&](int i) {
+		return double(ch->num_steps[i]) * std::max(1, ch->maxiters[i]) * (b.h.hdr[ch->model[i]].npairs + 1400.0);
+	};
+	if (may_speculate && spec == 1 && !forced)
+	{
+		// With more chains than that, the longest may speculate
+		// (critical_widths), each width a launch of its own.
+		std::vector<PlanChain> pc(static_cast<size_t>(n));
+		std::vector<int> all;
+		for (auto& kv : by_model)
+			all.push_back(kv.first);
+		const WavePlan largest = plan_for(b.h, all);
+		int per_cu[SPEC_WIDTHS];
+		for (int k = 0; k < SPEC_WIDTHS; k++)
+			per_cu[k] = spec_per_cu(largest, SPEC_WIDTH[k]);
+		for (Cls& k : cls)
+			if (!k.members.empty())
+			{
+				int maxper = 1, resident = 0;
+				for (auto& kv : k.members)
+					maxper = std::max(maxper, int(kv.second.size()));
+				occupancy_waves<T, S>(plan_for(b.h, k.models()), b.precision, variant, pdef, maxper, share, &resident);
+				for (auto& kv : k.members)
+					for (int i : kv.second)
+					{
+						pc[size_t(i)].cost = cost_of(i);
+						pc[size_t(i)].share[0] = 1.0 / std::max(1, resident);
+						for (int q = 0; q < SPEC_WIDTHS; q++)
+							pc[size_t(i)].share[1 + q] = per_cu[q] > 0 ? 1.0 / per_cu[q] : 0;
+					}
+			}
+		const std::vector<int> width = critical_widths(pc, prop.multiProcessorCount);
+		for (Cls& k : cls)
+			k.members.clear();
+		for (int i = 0; i < n; i++)
+		{
+			const int w = width[size_t(i)];
+			cls[w ? sgpu_ctx::NCLASS + w - 1 : class_of(ch->model[i])].members[ch->model[i]].push_back(i);
+			if (w)
+			{
+				hybrid = true;
+				spec = std::max(spec, SPEC_WIDTH[w - 1]);
+			}
+		}
+		// one stream each: the smallest size classes share a launch if there
+		// would be more than four
+		for (int k = 0; k + 1 < sgpu_ctx::NCLASS; k++)
+		{
+			int used = 0, next = k + 1;
+			for (const Cls& q : cls)
+				used += q.members.empty() ? 0 : 1;
+			while (next + 1 < sgpu_ctx::NCLASS && cls[next].members.empty())
+				next++;
+			if (used > sgpu_ctx::NCLASS && !cls[k].members.empty() && !cls[next].members.empty())
+			{
+				cls[next].members.insert(cls[k].members.begin(), cls[k].members.end());
+				cls[k].members.clear();
 			}
 		}
 	}
@@ -1636,9 +1791,16 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 	L.off_outx = take(size_t(MAX_POSES) * L.coord_stride * sizeof(T));
 	L.off_mc = take(L.atom_stride * sizeof(T));
 	L.off_ro = take(MAX_TREES * 3 * sizeof(T));
-	L.off_pbuf = take((sizeof(T) == 8 ? size_t(L.pair_stride) : 1) * sizeof(T));
-	// the ordered pair loop's scratch of a speculative chain's helper waves
-	L.off_hpbuf = take((sizeof(T) == 8 && spec > 1 ? size_t(spec - 1) * L.pair_stride : 1) * sizeof(T));
+	// the ordered search's pair energies, where they go through global memory
+	// (eval_deriv), and those of a speculative chain's helper waves
+	bool pair_scratch = false;
+	for (auto& kv : by_model)
+		pair_scratch = pair_scratch || (sizeof(T) == 8 && !b.h.hdr[size_t(kv.first)].one_ligand);
+	for (const Cls& k : cls)
+		if (!k.members.empty())
+			pair_scratch = pair_scratch || (sizeof(T) == 8 && !plan_for(b.h, k.models()).pair_lds);
+	L.off_pbuf = take((pair_scratch ? size_t(L.pair_stride) : 1) * sizeof(T));
+	L.off_hpbuf = take((pair_scratch && spec > 1 ? size_t(spec - 1) * L.pair_stride : 1) * sizeof(T));
 	L.off_ev = take(sizeof(int64_t));
 	// QuickVina 2's history: 5n points of n coordinates, n up to the batch's
 	// largest change size and at most 64 (chain_layout,
@@ -1666,38 +1828,36 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 		scal[0] = 0;
 		scal[1] = Real_host_max<S>();
 	}
-	const bool pdef = persist_default<T, S>(variant);
-	const int share = std::max(1, (n + prop.multiProcessorCount - 1) / prop.multiProcessorCount);
 	std::vector<int> block_model, slot_chain;
 	for (Cls& k : cls)
 	{
-		if (k.models.empty())
+		if (k.members.empty())
 			continue;
-		k.plan = plan_for(b.h, k.models);
+		const int ki = int(&k - cls);
+		const int width = ki >= sgpu_ctx::NCLASS ? SPEC_WIDTH[ki - sgpu_ctx::NCLASS] : hybrid ? 1 : spec;
+		k.plan = plan_for(b.h, k.models());
 		int maxper = 1;
-		for (int mi : k.models)
-			maxper = std::max(maxper, int(by_model[mi].size()));
+		for (auto& kv : k.members)
+			maxper = std::max(maxper, int(kv.second.size()));
 		// chains per workgroup by the occupancy rule
 		k.waves = occupancy_waves<T, S>(k.plan, b.precision, variant, pdef, maxper, share, &k.resident);
 		require(k.waves > 0, "chain state exceeds LDS");
 		// a probe's override, else the tuned plan of this class, where it fits
-		const int ki = int(&k - cls);
 		const sgpu_ctx::ClassPlan* cp = nullptr;
-		if (c->override_on[ki])
+		if (ki < sgpu_ctx::NCLASS && c->override_on[ki])
 			cp = &c->plan_override[ki];
-		else
+		else if (ki < sgpu_ctx::NCLASS)
 		{
 			auto it = c->tuned.find({b.precision, variant, ki});
 			if (it != c->tuned.end())
 				cp = &it->second;
 		}
-		if (spec > 1)
+		if (width > 1)
 		{
-			// one chain per workgroup of `spec` waves
-			k.waves = spec;
+			// one chain per workgroup of `width` waves
+			k.waves = width;
 			k.spec = true;
-			k.resident = spec * mc_blocks_per_cu<T, S>(spec, size_t(plan_bytes(k.plan, b.precision, spec)), variant,
-					false, true, k.plan.pair_lds);
+			k.resident = width * spec_per_cu(k.plan, width);
 		}
 		else if (cp && cp->waves >= 1 && cp->waves <= std::min(MAX_CHAINS_PER_GROUP, maxper) &&
 				plan_bytes(k.plan, b.precision, cp->waves) + LDS_STATIC <= LDS_LIMIT &&
@@ -1714,21 +1874,21 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 			std::fprintf(stderr,
 					"[sgpu] mc class %d: %zu models, %d waves/workgroup%s, %d LDS bytes/workgroup, %d resident "
 					"waves/CU (atoms %d, pairs %d, frames %d, change %d)\n",
-					int(&k - cls), k.models.size(), k.waves, k.spec ? " (one speculative chain)" : "", bytes,
+					ki, k.members.size(), k.waves, k.spec ? " (one speculative chain)" : "", bytes,
 					k.resident, k.plan.nmax, k.plan.pmax, k.plan.fmax,
 					k.plan.gmax);
 		}
-		for (int mi : k.models)
+		for (auto& kv : k.members)
 		{
-			const std::vector<int>& cs = by_model[mi];
+			const int mi = kv.first;
+			const std::vector<int>& cs = kv.second;
 			for (size_t s = 0; s < cs.size(); s += size_t(k.spec ? 1 : k.waves))
 			{
 				Blk bk{0, mi, {}};
 				for (size_t j = s; j < std::min(cs.size(), s + size_t(k.spec ? 1 : k.waves)); j++)
 				{
 					bk.chains.push_back(cs[j]);
-					bk.cost = std::max(bk.cost, double(ch->num_steps[cs[j]]) *
-									double(b.h.hdr[mi].npairs + 4 * b.h.hdr[mi].natoms));
+					bk.cost = std::max(bk.cost, cost_of(cs[j]));
 				}
 				k.blks.push_back(bk);
 			}
@@ -1805,7 +1965,7 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 			                   : int(k.blks.size());
 		}
 	DBuf dqueue;
-	const int nqueue = sgpu_ctx::NCLASS * (parts + 1);
+	const int nqueue = NGROUP * (parts + 1);
 	dqueue.alloc(size_t(nqueue) * sizeof(int));
 	// early stopping on the device (stop_agreeing, src/gpu/gpu_kernels_impl.cuh:
 	// 607-657): per model, its chains grouped by search unit, the units' count
@@ -1875,14 +2035,14 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 			// this part's launches on every stream
 			hip_check(hipEventRecord(c->part_start, c->stream), "event");
 			std::vector<hipStream_t> side;
-			for (int k = sgpu_ctx::NCLASS - 1; k >= 0; k--)
+			for (int k = NGROUP - 1; k >= 0; k--)
 			{
 				const Cls& cl = cls[k];
 				if (cl.blks.empty())
 					continue;
 				hipStream_t st = c->stream;
 				bool first = true;
-				for (int j = k + 1; j < sgpu_ctx::NCLASS; j++)
+				for (int j = k + 1; j < NGROUP; j++)
 					if (!cls[j].blks.empty())
 						first = false;
 				if (!first)
@@ -1891,7 +2051,7 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 					side.push_back(st);
 					hip_check(hipStreamWaitEvent(st, c->part_start, 0), "stream wait");
 				}
-				int* q = cl.persist ? dqueue.as<int>() + size_t(part) * sgpu_ctx::NCLASS + size_t(k) : nullptr;
+				int* q = cl.persist ? dqueue.as<int>() + size_t(part) * NGROUP + size_t(k) : nullptr;
 				hip_check(launch_mc<T, S>(ptrs<T>(b), ec, cl.plan, P, L, dchains.as<char>(), int(cl.blks.size()),
 								  cl.waves, dbm.as<int>() + cl.block_off, dsc.as<int>() + cl.slot_off,
 								  dsteps.as<int>(), dmax.as<int>(), lo, hi, parts, cl.grid, q, cl.spec, st),
