@@ -1139,6 +1139,7 @@ sgpu_status sgpu_build_grids(sgpu_ctx* c, int receptor_id, const sgpu_grid_dims*
 		a.fraction = c->tab.fraction;
 		a.nseg = c->tab.nseg;
 		std::vector<double> lo, hi;
+		std::vector<int> cell_point;
 		for (int d = 0; d < 3; d++)
 		{
 			a.cell_off[d] = int(std::floor(gd->begin[d] / 3.0));
@@ -1153,11 +1154,13 @@ sgpu_status sgpu_build_grids(sgpu_ctx* c, int receptor_id, const sgpu_grid_dims*
 		{
 			std::vector<double> l(a.cell_dim[d], 0), h(a.cell_dim[d], 0);
 			std::vector<char> seen(a.cell_dim[d], 0);
+			std::vector<int> npoints(size_t(a.cell_dim[d]) + 1, 0);
 			for (int i = 0; i <= gd->n[d]; i++)
 			{
 				const double cval = g->init[d] + g->factor_inv[d] * i;
 				const int cell = int(std::floor(cval / 3.0)) - a.cell_off[d];
 				require(cell >= 0 && cell < a.cell_dim[d], "probe outside the cell range");
+				npoints[size_t(cell) + 1]++; // (the points of a cell follow each other)
 				if (!seen[cell])
 				{
 					seen[cell] = 1;
@@ -1167,8 +1170,13 @@ sgpu_status sgpu_build_grids(sgpu_ctx* c, int receptor_id, const sgpu_grid_dims*
 			}
 			lo.insert(lo.end(), l.begin(), l.end());
 			hi.insert(hi.end(), h.begin(), h.end());
+			for (size_t k = 1; k < npoints.size(); k++)
+				npoints[k] += npoints[k - 1];
+			cell_point.insert(cell_point.end(), npoints.begin(), npoints.end());
 		}
-		DBuf dlo, dhi, dstart, datoms, dtypes;
+		DBuf dlo, dhi, dstart, datoms, dtypes, dpoint, drows;
+		upload(dpoint, cell_point, c->stream);
+		a.cell_point = dpoint.as<int>();
 		upload(dlo, lo, c->stream);
 		upload(dhi, hi, c->stream);
 		upload(dtypes, g->types, c->stream);
@@ -1197,7 +1205,9 @@ sgpu_status sgpu_build_grids(sgpu_ctx* c, int receptor_id, const sgpu_grid_dims*
 		g->charged = a.ncomp == 4;
 		if (g->charged)
 			g->qpoints.alloc(npts * ntypes * sizeof(double));
-		hip_check(launch_grid_points(a, g->points.as<double>(), g->qpoints.as<double>(), c->stream), "grid points");
+		drows.alloc(grid_row_bytes(a));
+		hip_check(launch_grid_points(a, drows.as<double>(), g->points.as<double>(), g->qpoints.as<double>(), c->stream),
+				"grid points");
 		const size_t ncell = size_t(g->dim[0] - 1) * (g->dim[1] - 1) * (g->dim[2] - 1) * ntypes * 8;
 		for (int q = 0; q < (g->charged ? 2 : 1); q++)
 		{

@@ -130,6 +130,7 @@ struct GridBuildArgs
 	double box_hi[3];
 	int* cell_start;       // [ncells + 1]
 	int* cell_atoms;       // sized by the count pass
+	const int* cell_point; // per axis [cell_dim + 1]: each cell's first point
 	int dim[3];            // grid points per axis
 	double init[3];
 	double factor_inv[3];
@@ -147,8 +148,10 @@ hipError_t launch_cell_fill(const GridBuildArgs& a, hipStream_t st);
 // the list entries of every cell as records, in both precisions
 hipError_t launch_cell_records(const double* xyz, const int* type, const int* cell_atoms, int total,
 		RecAtom<float>* rec32, RecAtom<double>* rec64, hipStream_t st);
-// points: [ntypes][npts]; qpoints: the charge maps, same layout (ncomp 4)
-hipError_t launch_grid_points(const GridBuildArgs& a, double* points, double* qpoints, hipStream_t st);
+// points: [ntypes][npts]; qpoints: the charge maps, same layout (ncomp 4);
+// rows: scratch of grid_row_bytes
+size_t grid_row_bytes(const GridBuildArgs& a);
+hipError_t launch_grid_points(const GridBuildArgs& a, double* rows, double* points, double* qpoints, hipStream_t st);
 template<typename T>
 hipError_t launch_grid_pack(const double* points, int ntypes, const int* dim, T* cells, hipStream_t st);
 
