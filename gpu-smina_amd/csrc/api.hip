@@ -1434,6 +1434,78 @@ __global__ void mc_queue_init(int* q, int n)
 		q[i] = 0;
 }
 
+// a chain's start state: its random stream, conf and energies, an empty
+// container and history.  One wave per chain.
+template<typename S>
+__global__ __launch_bounds__(WAVE) void mc_state_init(char* chains, ChainLayout L, const uint32_t* rng, const S* conf)
+{
+	const int i = int(blockIdx.x), lane = int(threadIdx.x);
+	char* p = chains + size_t(i) * L.bytes;
+	const uint32_t* r = rng + size_t(i) * 625;
+	uint32_t* mt = reinterpret_cast<uint32_t*>(p + L.off_mt);
+	for (int k = lane; k < MT_N; k += WAVE)
+		mt[k] = r[k];
+	S* tmp = reinterpret_cast<S*>(p + L.off_tmp);
+	for (int k = lane; k < L.conf_stride; k += WAVE)
+		tmp[k] = conf[size_t(i) * L.conf_stride + k];
+	if (lane == 0)
+	{
+		int* ints = reinterpret_cast<int*>(p + L.off_ints);
+		ints[0] = int(r[624]);
+		ints[1] = 0;
+		ints[2] = 0;
+		S* scal = reinterpret_cast<S*>(p + L.off_scal);
+		scal[0] = 0;
+		scal[1] = Real<S>::max();
+		*reinterpret_cast<int64_t*>(p + L.off_ev) = 0;
+		int* vis = reinterpret_cast<int*>(p + L.off_vs);
+		for (int k = 0; k < 3; k++)
+			vis[k] = 0;
+	}
+}
+
+// the chains' saved minima and evaluation counts
+__global__ void mc_counts(int n, const char* chains, ChainLayout L, int* count, int64_t* evals)
+{
+	const int i = int(blockIdx.x * blockDim.x + threadIdx.x);
+	if (i >= n)
+		return;
+	const char* p = chains + size_t(i) * L.bytes;
+	count[i] = reinterpret_cast<const int*>(p + L.off_ints)[1];
+	evals[i] = *reinterpret_cast<const int64_t*>(p + L.off_ev);
+}
+
+// where a chain's minima go in the packed results, and the sizes of one
+struct McPackRow
+{
+	size_t e, conf, x;
+	int conf_size, coords;
+};
+// one wave per chain
+template<typename T, typename S>
+__global__ __launch_bounds__(WAVE) void mc_pack(const char* chains, ChainLayout L, const McPackRow* rows, S* e, S* conf,
+		T* x)
+{
+	const int i = int(blockIdx.x), lane = int(threadIdx.x);
+	const char* p = chains + size_t(i) * L.bytes;
+	const McPackRow r = rows[i];
+	const int* ints = reinterpret_cast<const int*>(p + L.off_ints);
+	const S* oe = reinterpret_cast<const S*>(p + L.off_oute);
+	const S* oc = reinterpret_cast<const S*>(p + L.off_outc);
+	const T* ox = reinterpret_cast<const T*>(p + L.off_outx);
+	const int cnt = ints[1];
+	for (int k = 0; k < cnt; k++)
+	{
+		const size_t slot = size_t(ints[3 + k]);
+		if (lane == 0)
+			e[r.e + k] = oe[slot];
+		for (int j = lane; j < r.conf_size; j += WAVE)
+			conf[r.conf + size_t(k) * r.conf_size + j] = oc[slot * L.conf_stride + j];
+		for (int j = lane; j < r.coords; j += WAVE)
+			x[r.x + size_t(k) * r.coords + j] = ox[slot * L.coord_stride + j];
+	}
+}
+
 // stop_agreeing on the device, one thread per model: the best energy of
 // each search unit (the lowest over its chains' bests), the lowest of them,
 // and the units within eps of it; with at least need[m] agreeing, the model
@@ -1784,7 +1856,7 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 	L.coord_stride = 3 * hmax;
 	L.atom_stride = 3 * b.h.plan.nmax;
 	L.pair_stride = b.h.plan.pmax;
-	L.max_poses = MAX_POSES;
+	L.max_poses = p->num_saved_mins; // a container never holds more
 	size_t off = 0;
 	auto take = [&](size_t bytes) {
 		off = (off + 63) / 64 * 64;
@@ -1796,9 +1868,9 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 	L.off_ints = take((3 + MAX_POSES) * sizeof(int));
 	L.off_tmp = take(L.conf_stride * sizeof(S));
 	L.off_scal = take(2 * sizeof(S));
-	L.off_oute = take(MAX_POSES * sizeof(S));
-	L.off_outc = take(size_t(MAX_POSES) * L.conf_stride * sizeof(S));
-	L.off_outx = take(size_t(MAX_POSES) * L.coord_stride * sizeof(T));
+	L.off_oute = take(size_t(L.max_poses) * sizeof(S));
+	L.off_outc = take(size_t(L.max_poses) * L.conf_stride * sizeof(S));
+	L.off_outx = take(size_t(L.max_poses) * L.coord_stride * sizeof(T));
 	L.off_mc = take(L.atom_stride * sizeof(T));
 	L.off_ro = take(MAX_TREES * 3 * sizeof(T));
 	// the ordered search's pair energies, where they go through global memory
@@ -1821,23 +1893,6 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 	L.off_vb = take(size_t(10) * L.vis_n * sizeof(uint64_t));
 	L.off_vs = take(3 * sizeof(int));
 	L.bytes = (off + 63) / 64 * 64;
-	// initial chain state (the history empty: zeros)
-	std::vector<char> init(L.bytes * n, 0);
-	for (int i = 0; i < n; i++)
-	{
-		char* base = init.data() + L.bytes * i;
-		std::memcpy(base + L.off_mt, ch->rng + size_t(i) * 625, MT_N * sizeof(uint32_t));
-		int* ints = reinterpret_cast<int*>(base + L.off_ints);
-		ints[0] = int(ch->rng[size_t(i) * 625 + 624]);
-		ints[1] = 0;
-		ints[2] = 0;
-		S* tmp = reinterpret_cast<S*>(base + L.off_tmp);
-		for (int k = 0; k < b.h.hdr[ch->model[i]].conf_size; k++)
-			tmp[k] = S(ch->conf[size_t(i) * ch->conf_stride + k]);
-		S* scal = reinterpret_cast<S*>(base + L.off_scal);
-		scal[0] = 0;
-		scal[1] = Real_host_max<S>();
-	}
 	std::vector<int> block_model, slot_chain;
 	for (Cls& k : cls)
 	{
@@ -1913,8 +1968,23 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 				slot_chain.push_back(k.spec ? bk.chains[0] : j < int(bk.chains.size()) ? bk.chains[j] : -1);
 		}
 	}
-	DBuf dchains, dbm, dsc, dsteps, dmax;
-	upload(dchains, init, c->stream);
+	DBuf dchains, dbm, dsc, dsteps, dmax, drng, dconf;
+	dchains.alloc(L.bytes * size_t(n));
+	{
+		// the chains' states are written on the device from their start confs
+		// and random streams
+		std::vector<S> conf(size_t(n) * L.conf_stride, S(0));
+		for (int i = 0; i < n; i++)
+			for (int k = 0; k < b.h.hdr[ch->model[i]].conf_size; k++)
+				conf[size_t(i) * L.conf_stride + k] = S(ch->conf[size_t(i) * ch->conf_stride + k]);
+		upload(dconf, conf, c->stream);
+		drng.alloc(size_t(n) * 625 * sizeof(uint32_t));
+		hip_check(hipMemcpyAsync(drng.p, ch->rng, size_t(n) * 625 * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream),
+				"upload");
+		hipLaunchKernelGGL((mc_state_init<S>), dim3(n), dim3(WAVE), 0, c->stream, dchains.as<char>(), L,
+				drng.as<uint32_t>(), dconf.as<S>());
+		hip_check(hipGetLastError(), "chain states");
+	}
 	upload(dbm, block_model, c->stream);
 	upload(dsc, slot_chain, c->stream);
 	upload(dsteps, std::vector<int>(ch->num_steps, ch->num_steps + n), c->stream);
@@ -2121,30 +2191,58 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 	tm.stop();
 	if (c->progress_fn)
 		c->progress_fn(c->progress_user, 1.0);
-	hip_check(hipMemcpyAsync(init.data(), dchains.p, init.size(), hipMemcpyDeviceToHost, c->stream), "download");
+	// the results: counts first, then the saved minima of all chains packed in
+	// their own sizes, best first
+	DBuf dcnt, dev, doff, dpe, dpc, dpx;
+	dcnt.alloc(size_t(n) * sizeof(int));
+	dev.alloc(size_t(n) * sizeof(int64_t));
+	hipLaunchKernelGGL(mc_counts, dim3(unsigned((n + 255) / 256)), dim3(256), 0, c->stream, n, dchains.as<char>(), L,
+			dcnt.as<int>(), dev.as<int64_t>());
+	hip_check(hipGetLastError(), "counts");
+	std::vector<int64_t> ev(n);
+	hip_check(hipMemcpyAsync(out->count, dcnt.p, size_t(n) * sizeof(int), hipMemcpyDeviceToHost, c->stream), "download");
+	hip_check(hipMemcpyAsync(ev.data(), dev.p, size_t(n) * sizeof(int64_t), hipMemcpyDeviceToHost, c->stream), "download");
 	hip_check(hipStreamSynchronize(c->stream), "mc");
+	std::vector<McPackRow> rows(static_cast<size_t>(n));
+	size_t ne = 0, nc = 0, nx = 0;
 	for (int i = 0; i < n; i++)
 	{
-		const char* base = init.data() + L.bytes * i;
 		const ModelHdr& h = b.h.hdr[ch->model[i]];
-		const int* ints = reinterpret_cast<const int*>(base + L.off_ints);
-		const int cnt = std::min(ints[1], out->max_poses);
-		const S* oe = reinterpret_cast<const S*>(base + L.off_oute);
-		const S* oc = reinterpret_cast<const S*>(base + L.off_outc);
-		const T* ox = reinterpret_cast<const T*>(base + L.off_outx);
-		out->count[i] = cnt;
-		for (int k = 0; k < cnt; k++)
+		rows[size_t(i)] = {ne, nc, nx, h.conf_size, 3 * h.nheavy};
+		ne += size_t(out->count[i]);
+		nc += size_t(out->count[i]) * h.conf_size;
+		nx += size_t(out->count[i]) * 3 * h.nheavy;
+	}
+	std::unique_ptr<S[]> pe(new S[std::max<size_t>(1, ne)]), pc(new S[std::max<size_t>(1, nc)]);
+	std::unique_ptr<T[]> px(new T[std::max<size_t>(1, nx)]);
+	if (ne > 0)
+	{
+		upload(doff, rows, c->stream);
+		dpe.alloc(ne * sizeof(S));
+		dpc.alloc(std::max<size_t>(1, nc) * sizeof(S));
+		dpx.alloc(std::max<size_t>(1, nx) * sizeof(T));
+		hipLaunchKernelGGL((mc_pack<T, S>), dim3(n), dim3(WAVE), 0, c->stream, dchains.as<char>(), L, doff.as<McPackRow>(),
+				dpe.as<S>(), dpc.as<S>(), dpx.as<T>());
+		hip_check(hipGetLastError(), "pack");
+		hip_check(hipMemcpyAsync(pe.get(), dpe.p, ne * sizeof(S), hipMemcpyDeviceToHost, c->stream), "download");
+		hip_check(hipMemcpyAsync(pc.get(), dpc.p, nc * sizeof(S), hipMemcpyDeviceToHost, c->stream), "download");
+		hip_check(hipMemcpyAsync(px.get(), dpx.p, nx * sizeof(T), hipMemcpyDeviceToHost, c->stream), "download");
+		hip_check(hipStreamSynchronize(c->stream), "mc");
+	}
+	for (int i = 0; i < n; i++)
+	{
+		const McPackRow& r = rows[size_t(i)];
+		for (int k = 0; k < out->count[i]; k++)
 		{
-			const int slot = ints[3 + k];
-			out->e[size_t(i) * out->max_poses + k] = double(oe[slot]);
-			for (int j = 0; j < h.conf_size; j++)
-				out->conf[(size_t(i) * out->max_poses + k) * out->conf_stride + j] = double(oc[size_t(slot) * L.conf_stride + j]);
-			for (int j = 0; j < 3 * h.nheavy; j++)
-				out->coords[(size_t(i) * out->max_poses + k) * out->coord_stride + j] =
-						double(ox[size_t(slot) * L.coord_stride + j]);
+			const size_t row = size_t(i) * out->max_poses + k;
+			out->e[row] = double(pe[r.e + k]);
+			for (int j = 0; j < r.conf_size; j++)
+				out->conf[row * out->conf_stride + j] = double(pc[r.conf + size_t(k) * r.conf_size + j]);
+			for (int j = 0; j < r.coords; j++)
+				out->coords[row * out->coord_stride + j] = double(px[r.x + size_t(k) * r.coords + j]);
 		}
 		if (out->evals)
-			out->evals[i] = *reinterpret_cast<const int64_t*>(base + L.off_ev);
+			out->evals[i] = ev[size_t(i)];
 	}
 }
 

@@ -8,6 +8,9 @@
 
 #include <algorithm>
 #include <chrono>
+#include <thread>
+#include <system_error>
+#include <exception>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -1263,24 +1266,69 @@ void GpuDocking::fp64_errors(DockJob* const* jobs, size_t nj, int batch, int cst
 	}
 }
 
+// f(0) .. f(n - 1) on up to 16 threads (one for small n), in runs of
+// neighbouring indices; the exception of the lowest index that throws is
+// rethrown
+template<typename F>
+static void parallel_for(size_t n, size_t grain, F&& f)
+{
+	const size_t hw = std::max(1u, std::thread::hardware_concurrency());
+	const size_t nt = std::min({size_t(16), hw, n / std::max<size_t>(1, grain)});
+	if (nt < 2)
+	{
+		for (size_t i = 0; i < n; i++)
+			f(i);
+		return;
+	}
+	std::vector<std::exception_ptr> failed(nt);
+	auto part = [&](size_t t) {
+		try
+		{
+			for (size_t i = n * t / nt; i < n * (t + 1) / nt; i++)
+				f(i);
+		}
+		catch (...)
+		{
+			failed[t] = std::current_exception();
+		}
+	};
+	std::vector<std::thread> threads;
+	size_t started = 1;
+	try
+	{
+		for (; started < nt; started++)
+			threads.emplace_back(part, started);
+	}
+	catch (const std::system_error&)
+	{
+		// no more threads: this one takes the parts that have none
+	}
+	part(0);
+	for (size_t t = started; t < nt; t++)
+		part(t);
+	for (std::thread& t : threads)
+		t.join();
+	for (const std::exception_ptr& e : failed)
+		if (e)
+			std::rethrow_exception(e);
+}
+
 void GpuDocking::dock_sub(DockJob* const* jobs, size_t nj, double budget)
 {
 	if (nj == 0)
 		return;
 	const auto t0 = std::chrono::steady_clock::now();
 	const int prec = s_.precision;
-	std::vector<FlatModel> fms;
+	std::vector<FlatModel> fms(nj);
 	std::vector<int> types;
+	parallel_for(nj, 16, [&](size_t j) { fms[j] = flatten(*jobs[j]->m); });
 	for (size_t j = 0; j < nj; j++)
-	{
-		fms.push_back(flatten(*jobs[j]->m));
-		for (int a = 0; a < fms.back().view.natoms; a++)
+		for (int a = 0; a < fms[j].view.natoms; a++)
 		{
-			const int t = fms.back().atom_type[a];
+			const int t = fms[j].atom_type[a];
 			if (!is_hydrogen_type(t) && std::find(types.begin(), types.end(), t) == types.end())
 				types.push_back(t);
 		}
-	}
 	ensure_grids(types);
 	std::vector<sgpu_flat_model> views;
 	for (auto& f : fms)
@@ -1296,9 +1344,7 @@ void GpuDocking::dock_sub(DockJob* const* jobs, size_t nj, double budget)
 	}
 	// with split n, n chains per exhaustiveness unit, each with 1/n of the
 	// steps (add_chains and chain_steps, src/gpu/gpu_docking.cpp:200-220)
-	std::vector<int> cmodel, csteps, citers, cunit;
-	std::vector<double> cconf;
-	std::vector<uint32_t> crng;
+	std::vector<int> cmodel, csteps, citers, cunit, cseed;
 	std::vector<size_t> first(nj + 1, 0);
 	std::vector<SearchParams> sp;
 	size_t tasks = 0;
@@ -1316,20 +1362,20 @@ void GpuDocking::dock_sub(DockJob* const* jobs, size_t nj, double budget)
 		const int steps = std::max(1, int(std::ceil(double(sp[j].num_steps) * fraction / double(split))));
 		for (int t = 0; t < exh * split; t++)
 		{
-			const int seed = random_int(0, 1000000, g);
-			std::vector<double> conf(cstride, 0.0);
-			std::vector<uint32_t> st(625);
-			make_chain(fms[j], uint32_t(seed), gd_, conf.data(), st.data());
+			cseed.push_back(random_int(0, 1000000, g));
 			cmodel.push_back(int(j));
 			csteps.push_back(steps);
 			citers.push_back(sp[j].maxiters);
 			cunit.push_back(t / split);
-			cconf.insert(cconf.end(), conf.begin(), conf.end());
-			crng.insert(crng.end(), st.begin(), st.end());
 		}
 	}
 	first[nj] = cmodel.size();
 	const int nchains = int(cmodel.size());
+	std::vector<double> cconf(size_t(nchains) * cstride, 0.0);
+	std::vector<uint32_t> crng(size_t(nchains) * 625);
+	parallel_for(size_t(nchains), 128, [&](size_t c) {
+		make_chain(fms[size_t(cmodel[c])], uint32_t(cseed[c]), gd_, cconf.data() + c * cstride, crng.data() + c * 625);
+	});
 	sgpu_chains ch{nchains, cmodel.data(), cconf.data(), cstride, crng.data(), csteps.data(), citers.data(),
 			cunit.data()};
 	sgpu_mc_params mp{};
@@ -1358,10 +1404,11 @@ void GpuDocking::dock_sub(DockJob* const* jobs, size_t nj, double budget)
 	}
 	const int maxp = mp.num_saved_mins;
 	std::vector<int> cnt(nchains);
-	std::vector<double> oe(size_t(nchains) * maxp), oc(size_t(nchains) * maxp * cstride),
-			ox(size_t(nchains) * maxp * hstride);
+	// not initialised: only the poses that the chains saved are written and read
+	std::unique_ptr<double[]> oe(new double[size_t(nchains) * maxp]), oc(new double[size_t(nchains) * maxp * cstride]),
+			ox(new double[size_t(nchains) * maxp * hstride]);
 	std::vector<int64_t> evals(nchains, 0);
-	sgpu_chain_results res{maxp, cstride, hstride, cnt.data(), oe.data(), oc.data(), ox.data(), evals.data()};
+	sgpu_chain_results res{maxp, cstride, hstride, cnt.data(), oe.get(), oc.get(), ox.get(), evals.data()};
 	if (tune_report_)
 	{
 		// a tuning call: probe the launch plans on these chains, search nothing
@@ -1374,8 +1421,7 @@ void GpuDocking::dock_sub(DockJob* const* jobs, size_t nj, double budget)
 	std::vector<int> pose_model, pose_iters;
 	std::vector<double> pose_conf;
 	std::vector<std::pair<size_t, size_t>> pose_ref;
-	for (size_t j = 0; j < nj; j++)
-	{
+	parallel_for(nj, 4, [&](size_t j) {
 		auto& out = jobs[j]->out;
 		out.clear();
 		jobs[j]->evals = 0;
@@ -1387,11 +1433,15 @@ void GpuDocking::dock_sub(DockJob* const* jobs, size_t nj, double budget)
 				Pose p;
 				const size_t slot = c * maxp + k;
 				p.e = oe[slot];
-				p.c.assign(oc.begin() + slot * cstride, oc.begin() + slot * cstride + fms[j].view.conf_size);
-				p.coords.assign(ox.begin() + slot * hstride, ox.begin() + slot * hstride + 3 * fms[j].nheavy);
+				p.c.assign(oc.get() + slot * cstride, oc.get() + slot * cstride + fms[j].view.conf_size);
+				p.coords.assign(ox.get() + slot * hstride, ox.get() + slot * hstride + 3 * fms[j].nheavy);
 				add_to_output_container(out, p, 2, size_t(sp[j].num_saved_mins));
 			}
 		}
+	});
+	for (size_t j = 0; j < nj; j++)
+	{
+		const auto& out = jobs[j]->out;
 		for (size_t k = 0; k < out.size(); k++)
 		{
 			pose_model.push_back(int(j));
@@ -1503,8 +1553,7 @@ void GpuDocking::dock_sub(DockJob* const* jobs, size_t nj, double budget)
 			}
 		}
 	}
-	for (size_t j = 0; j < nj; j++)
-	{
+	parallel_for(nj, 16, [&](size_t j) {
 		auto& out = jobs[j]->out;
 		std::stable_sort(out.begin(), out.end(), [](const Pose& a, const Pose& b) { return a.e < b.e; });
 		// remove_redundant with --min_rmsd_filter (src/main/main.cpp:204-210, :276)
@@ -1520,7 +1569,7 @@ void GpuDocking::dock_sub(DockJob* const* jobs, size_t nj, double budget)
 			fin.push_back(tmp[i]);
 		}
 		out.swap(fin);
-	}
+	});
 	fp64_errors(jobs, nj, batch, cstride);
 	sgpu_release_models(ctx_, batch);
 	const double secs = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
