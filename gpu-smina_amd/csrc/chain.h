@@ -405,7 +405,7 @@ struct Searcher
 		{
 			++evals;
 			T ge_t;
-			const S fe = S(eval_deriv<T, BK, SPL, PS>(m, ec, W, pbuf, T(xe), ge_t));
+			const S fe = S(eval_deriv<T, BK, SPL, PS, Real<T>::ordered || !SPEC>(m, ec, W, pbuf, T(xe), ge_t));
 			const S ge = S(ge_t);
 			helper_last = false;
 			bool begin = false;
@@ -655,7 +655,7 @@ __device__ inline void spec_helper(const MV<T>& m, const EvalCtx<T>& ec, WaveMem
 		const S xe = conf_increment(m, SM, alpha);
 		lsync();
 		T g;
-		const S f = S(eval_deriv<T, BK_MAPS, SPL, PS>(m, ev, W, pbuf, T(xe), g));
+		const S f = S(eval_deriv<T, BK_MAPS, SPL, PS, Real<T>::ordered>(m, ev, W, pbuf, T(xe), g));
 		S* r = L.res + rank * SPEC_RS;
 		if (lane == 0)
 			r[0] = f;

@@ -91,3 +91,15 @@ def test_fp64_chain_with_pairs_past_lds(ctx):
                                   coord_stride=3 * f.nheavy)
     eo, co, xo, evo = o.mc_chain(ids[0], sg.mc_params(), 2, 8, c0, s0)
     assert cnt[0] == len(eo) and np.array_equal(e[0, :cnt[0]], eo) and ev[0] == evo
+
+
+@pytest.mark.parametrize("passes", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("prec", [sg.FP64, sg.FP32], ids=["fp64", "fp32"])
+def test_pair_batches(ctx, passes, prec):
+    """every mix of whole batches of 4 passes and a shorter last one"""
+    for seed in range(1, 400):
+        lig = sg.Mol.ligand(seed, 10 + seed % 30, 1 + seed % 5 if seed % 30 > 12 else 1)
+        f = sg.Flat(lig)
+        if (f.npairs + 63) // 64 == passes:
+            return check(ctx, lig, f, prec, 0)
+    raise AssertionError("no such ligand")
