@@ -1711,8 +1711,7 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 	// Launch plan.  Ligands fall into size classes by pair count; each class
 	// gets its own LDS plan (sized for its largest member) and runs on its own
 	// stream, concurrently with the others.  Within a class, workgroups hold
-	// `waves` chains of one ligand (the largest power of two up to 8 that the
-	// chains per ligand and 160 KB of LDS allow), costliest first.
+	// `waves` chains of one ligand (occupancy_waves), costliest first.
 	std::map<int, std::vector<int>> by_model;
 	for (int i = 0; i < n; i++)
 		by_model[ch->model[i]].push_back(i);

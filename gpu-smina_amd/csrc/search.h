@@ -555,8 +555,7 @@ __device__ __forceinline__ void set_conf(const MV<T>& m, WaveMem<T>& W, T x_lane
 }
 
 // what a wave's LDS holds throughout a kernel: the hydrogens' forces (FP64),
-// the fixed atoms
-// (flexible-residue atoms that do not move) after the movable ones in the
+// the fixed atoms (flexible-residue atoms that do not move) after the movable ones in the
 // coordinate array, and the pair slot of the lists' padding, no force
 template<typename T, bool PS>
 __device__ inline void init_wave(const MV<T>& m, WaveMem<T>& W)
@@ -578,7 +577,6 @@ __device__ inline void init_wave(const MV<T>& m, WaveMem<T>& W)
 // precalculate_splines::eval_deriv, one component, no slow terms
 // (src/lib/precalculate.h:418-450) with Spline::eval_deriv
 // (src/lib/splines.h:103-121): the spline at r = sqrt(r2), its derivative
-// over r
 // over r, in FP64 (the FP32 search rounds the results)
 template<typename T>
 __device__ inline void spline_deriv(const TablePtrs<T>& tab, int tri, T r2, T& e, T& dor)

@@ -217,7 +217,7 @@ sgpu_status sgpu_device_info(sgpu_ctx* ctx, char* name, int name_len, int* cus);
 sgpu_status sgpu_device_memory(sgpu_ctx* ctx, size_t* free_bytes, size_t* total_bytes);
 /* Monte Carlo chains of this precision the device holds at once (one per
  * wave, as the occupancy calculator gives it from the search kernel's
- * registers): EngineBase::capacity, src/gpu/gpu_docking.cpp:223-226 */
+ * registers, at most two waves per SIMD): EngineBase::capacity, src/gpu/gpu_docking.cpp:223-226 */
 sgpu_status sgpu_mc_capacity(sgpu_ctx* ctx, int precision, int* chains);
 
 /* DeviceTables::upload (src/gpu/gpu_device.cu:71-90) */
