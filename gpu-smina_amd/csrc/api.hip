@@ -322,6 +322,7 @@ void pack_batch(const sgpu_flat_model* ms, int n, HostBatch& B)
 		auto mark = [&](int& off) { off = int(I.size()); };
 		// neighbour lists in evaluation (pair) order
 		std::vector<std::vector<int>> lists(m.natoms);
+		bool hydrogen_pair = false;
 		for (int p = 0; p < m.npairs; p++)
 		{
 			const int a = m.pair_a[p], b = m.pair_b[p];
@@ -329,6 +330,7 @@ void pack_batch(const sgpu_flat_model* ms, int n, HostBatch& B)
 			const int tri = m.pair_tri[p];
 			require(tri >= 0 && tri < SGPU_NUM_TYPE_PAIRS, "pair type index out of range");
 			require(tri == tri_index_permissive(m.atom_type[a], m.atom_type[b]), "pair table index disagrees with types");
+			hydrogen_pair = hydrogen_pair || is_hydrogen_type(m.atom_type[a]) || is_hydrogen_type(m.atom_type[b]);
 			lists[a].push_back(make_code(b, p + 1));
 			if (b < m.natoms)
 				lists[b].push_back(make_code(a, p + 1));
@@ -433,6 +435,7 @@ void pack_batch(const sgpu_flat_model* ms, int n, HostBatch& B)
 				++nh;
 			}
 		h.nheavy = nh;
+		h.heavy_lanes = m.natoms > WAVE && nh >= 1 && nh <= WAVE && !hydrogen_pair;
 		// trees
 		std::vector<int> troot(m.ntrees, -1), tab(m.ntrees, m.natoms), tae(m.ntrees, 0), tn(m.ntrees, 0);
 		for (int f = 0; f < m.nframes; f++)

@@ -142,6 +142,7 @@ struct ModelHdr
 	int path_ok; // every root-to-frame path has at most MAX_PATH frames
 	int ncodes;
 	int one_ligand; // one ligand whose pairs are all those after the other pairs
+	int heavy_lanes; // over 64 movable atoms, 1..64 of them heavy, no hydrogen in a pair (eval_deriv)
 	int iblob_off, iblob_len; // in the batch int blob
 	int tblob_off, tblob_len; // in the batch real blob
 	// offsets inside the int blob (the movable atoms' records at 0)

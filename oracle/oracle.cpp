@@ -2556,6 +2556,7 @@ void orc_model_pairs(orc_ctx* c, int model, int* a, int* b, int* list)
 			list[k++] = 0;
 		}
 }
+void orc_add_ligand_pair(orc_ctx* c, int model, int a, int b) { c->c.models[model]->lig_pairs[0].push_back({a, b}); }
 double orc_num_tors(orc_ctx* c, int model) { return c->c.models[model]->num_tors; }
 double orc_eval_deriv(orc_ctx* c, int model, int backend, double slope, const double* v, const double* conf,
 		double* g, double* coords)

@@ -74,6 +74,9 @@ void orc_model_info(orc_ctx* c, int model, int* info);
 void orc_initial_conf(orc_ctx* c, int model, double* conf);
 /* the pairs in evaluation order: a, b, list (0 ligand, 2 other) */
 void orc_model_pairs(orc_ctx* c, int model, int* a, int* b, int* list);
+/* one more ligand pair (of ligand 0, evaluated last), whatever its types:
+ * a model that initialize_pairs would not make (hydrogen pairs) */
+void orc_add_ligand_pair(orc_ctx* c, int model, int a, int b);
 double orc_num_tors(orc_ctx* c, int model);
 
 /* model::eval_deriv (src/lib/model.cpp:969-983); backend 0 = cache (grids),

@@ -47,6 +47,7 @@ def _load():
         "orc_model_info": (None, [vp, C.c_int, I32P]),
         "orc_initial_conf": (None, [vp, C.c_int, F64P]),
         "orc_model_pairs": (None, [vp, C.c_int, I32P, I32P, I32P]),
+        "orc_add_ligand_pair": (None, [vp, C.c_int, C.c_int, C.c_int]),
         "orc_num_tors": (C.c_double, [vp, C.c_int]),
         "orc_eval_deriv": (C.c_double, [vp, C.c_int, C.c_int, C.c_double, F64P, F64P, F64P, F64P]),
         "orc_eval": (C.c_double, [vp, C.c_int, C.c_double, F64P, F64P]),
@@ -229,6 +230,9 @@ class Oracle:
         a, b, lst = (np.zeros(n, np.int32) for _ in range(3))
         lib.orc_model_pairs(self.h, m, _p(a, I32P), _p(b, I32P), _p(lst, I32P))
         return a, b, lst
+
+    def add_ligand_pair(self, m, a, b):
+        lib.orc_add_ligand_pair(self.h, m, a, b)
 
     def num_tors(self, m):
         return lib.orc_num_tors(self.h, m)
