@@ -892,7 +892,7 @@ __device__ __forceinline__ double row_ordered_add(double acc, double v)
 	asm("s_nop 1\n\t" SGPU_ROW_ADD(0) SGPU_ROW_ADD(1) SGPU_ROW_ADD(2) SGPU_ROW_ADD(3) SGPU_ROW_ADD(4) SGPU_ROW_ADD(5)
 					SGPU_ROW_ADD(6) SGPU_ROW_ADD(7) SGPU_ROW_ADD(8) SGPU_ROW_ADD(9) SGPU_ROW_ADD(10) SGPU_ROW_ADD(11)
 							SGPU_ROW_ADD(12) SGPU_ROW_ADD(13) SGPU_ROW_ADD(14) SGPU_ROW_ADD(15)
-			: "+v"(acc)
+			: "+&v"(acc) // (not v's register: every instruction reads v)
 			: "v"(v), "v"(1.0));
 #undef SGPU_ROW_ADD
 	return acc;
