@@ -255,7 +255,6 @@ struct sgpu_ctx
 namespace
 {
 
-constexpr int LDS_LIMIT = 160 * 1024;
 constexpr int LDS_STATIC = 64; // the persistent Monte Carlo kernel's own LDS (its work item)
 
 // the LDS plan that fits every listed model of a packed batch
@@ -1828,10 +1827,28 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 		{
 			const int w = width[size_t(i)];
 			cls[w ? sgpu_ctx::NCLASS + w - 1 : class_of(ch->model[i])].members[ch->model[i]].push_back(i);
-			if (w)
+		}
+		for (int w = 0; w < SPEC_WIDTHS; w++)
+		{
+			// A group's plan is its own: in FP64 it holds its pairs in LDS
+			// where the plan of all models, the shares' plan, does not, and
+			// may then not fit at its width.  The models with the most pairs
+			// leave such a group and run alone.
+			std::map<int, std::vector<int>>& group = cls[sgpu_ctx::NCLASS + w].members;
+			while (!group.empty() && spec_per_cu(plan_for(b.h, cls[sgpu_ctx::NCLASS + w].models()), SPEC_WIDTH[w]) < 1)
+			{
+				auto most = std::max_element(group.begin(), group.end(), [&](const auto& x, const auto& y) {
+					return b.h.hdr[size_t(x.first)].npairs < b.h.hdr[size_t(y.first)].npairs;
+				});
+				std::vector<int>& alone = cls[class_of(most->first)].members[most->first];
+				alone.insert(alone.end(), most->second.begin(), most->second.end());
+				std::sort(alone.begin(), alone.end());
+				group.erase(most);
+			}
+			if (!group.empty())
 			{
 				hybrid = true;
-				spec = std::max(spec, SPEC_WIDTH[w - 1]);
+				spec = std::max(spec, SPEC_WIDTH[w]);
 			}
 		}
 		// one stream each: the smallest size classes share a launch if there

@@ -41,6 +41,7 @@ namespace sgpu
 {
 
 constexpr int WAVE = 64;
+constexpr int LDS_LIMIT = 160 * 1024; // a workgroup's LDS
 constexpr int MAX_ATOMS = 255;    // movable + fixed atoms per model (8-bit partner field)
 constexpr int MAX_PAIRS = 8191;   // 13-bit pair field
 constexpr int MAX_FRAMES = 64;
