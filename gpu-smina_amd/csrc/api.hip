@@ -1142,6 +1142,7 @@ sgpu_status sgpu_build_grids(sgpu_ctx* c, int receptor_id, const sgpu_grid_dims*
 		a.nseg = c->tab.nseg;
 		std::vector<double> lo, hi;
 		std::vector<int> cell_point;
+		a.cell_tiles = 1;
 		for (int d = 0; d < 3; d++)
 		{
 			a.cell_off[d] = int(std::floor(gd->begin[d] / 3.0));
@@ -1172,6 +1173,7 @@ sgpu_status sgpu_build_grids(sgpu_ctx* c, int receptor_id, const sgpu_grid_dims*
 			}
 			lo.insert(lo.end(), l.begin(), l.end());
 			hi.insert(hi.end(), h.begin(), h.end());
+			a.cell_tiles *= (*std::max_element(npoints.begin(), npoints.end()) + 3) / 4;
 			for (size_t k = 1; k < npoints.size(); k++)
 				npoints[k] += npoints[k - 1];
 			cell_point.insert(cell_point.end(), npoints.begin(), npoints.end());

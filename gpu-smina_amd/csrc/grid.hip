@@ -10,7 +10,7 @@
  *    builds (src/lib/szv_grid.h:100-130), degenerate where a probe lies on a
  *    3 A boundary.  Count pass, scan, ordered fill (one workgroup per cell,
  *    prefix sums keep receptor order).
- * 2. points: one workgroup per cell, whose list it stages in LDS as records;
+ * 2. points: the workgroups of a cell stage its list in LDS as records;
  *    each wave sums tiles of 4 x 4 x 4 of the cell's points over the list
  *    (FP64, in list order) for every needed ligand type.  The linear tables
  *    are first repacked to one row per receptor type and knot holding all
@@ -183,6 +183,7 @@ __global__ __launch_bounds__(256) void type_rows_kernel(const double* fast, int 
 
 constexpr int POINT_WAVES = 4;
 constexpr int POINT_LIST = 512; // records in LDS at once
+constexpr int MAX_SPLIT = 256;  // workgroups of a cell
 enum PointTables
 {
 	POINTS_LINEAR = 0,
@@ -190,12 +191,16 @@ enum PointTables
 	POINTS_SPLINE = 2
 };
 
-// One cell's points.  Bound by the table rows' gathers: a tile's 64 points
-// walk the same list (broadcast reads from LDS) and skip an atom none of them
-// reaches; with a thread per x-fastest point (nine lists a wave, an index, a
-// position and a type load per entry, a gather per ligand type) the 531,441
-// points of a 30 A box took 1,676 us for 8 types, now 345 us (four entries' rows in
-// flight at once: no faster).
+// One cell's points, its tiles split over gridDim.y workgroups.  Bound by the
+// table rows' gathers: a tile's 64 points walk the same list (broadcast reads
+// from LDS) and skip an atom none of them reaches.  A thread per x-fastest
+// point (nine lists a wave, an index, a position and a type load per entry, a
+// gather per ligand type) took 1,676 us for the 531,441 points and 8 types of
+// a 30 A box, this 345 us with all of a cell's tiles in one workgroup (four
+// entries' rows in flight at once: no faster).  With one workgroup a cell, a
+// box of few cells or of many points a cell left most of the device idle: a
+// whole build of a 12 A box at 0.1 A took 4.7 ms (linear) and 40 ms (spline),
+// of a 22.5 A box at 0.375 A with splines 1.77 ms; split, 1.1, 2.6 and 1.27 ms.
 template<int NT, int KIND>
 __global__ __launch_bounds__(64 * POINT_WAVES) void grid_points_kernel(GridBuildArgs a, const double* rows,
 		double* points, double* qpoints)
@@ -221,7 +226,7 @@ __global__ __launch_bounds__(64 * POINT_WAVES) void grid_points_kernel(GridBuild
 	const int lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6;
 	const size_t npts = size_t(a.dim[0]) * a.dim[1] * a.dim[2];
 	int staged = -1; // the list's part in LDS
-	for (int t0 = 0; t0 < ntiles; t0 += POINT_WAVES)
+	for (int t0 = int(blockIdx.y) * POINT_WAVES; t0 < ntiles; t0 += int(gridDim.y) * POINT_WAVES)
 	{
 		const int tile = t0 + wave;
 		const int px = 4 * (tile % tiles[0]) + (lane & 3);
@@ -407,8 +412,11 @@ hipError_t launch_grid_points(const GridBuildArgs& a, double* rows, double* poin
 	          : nt == 4      ? grid_points_kernel<4, POINTS_LINEAR>
 	          : nt == 8      ? grid_points_kernel<8, POINTS_LINEAR>
 	                         : grid_points_kernel<16, POINTS_LINEAR>;
-	hipLaunchKernelGGL(fn, dim3(unsigned(a.cell_dim[0] * a.cell_dim[1] * a.cell_dim[2])), dim3(64 * POINT_WAVES), 0, st, a,
-			rows, points, qpoints);
+	const int ncells = a.cell_dim[0] * a.cell_dim[1] * a.cell_dim[2];
+	// a tile per wave, so that a few cells of many points fill the device, too
+	const int split = (a.cell_tiles + POINT_WAVES - 1) / POINT_WAVES;
+	hipLaunchKernelGGL(fn, dim3(unsigned(ncells), unsigned(split < MAX_SPLIT ? split : MAX_SPLIT)), dim3(64 * POINT_WAVES),
+			0, st, a, rows, points, qpoints);
 	return hipGetLastError();
 }
 

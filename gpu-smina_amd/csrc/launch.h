@@ -131,6 +131,7 @@ struct GridBuildArgs
 	int* cell_start;       // [ncells + 1]
 	int* cell_atoms;       // sized by the count pass
 	const int* cell_point; // per axis [cell_dim + 1]: each cell's first point
+	int cell_tiles;        // tiles of 4 x 4 x 4 points that a cell has at most
 	int dim[3];            // grid points per axis
 	double init[3];
 	double factor_inv[3];
