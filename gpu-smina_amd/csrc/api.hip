@@ -241,6 +241,10 @@ struct sgpu_ctx
 	std::map<std::array<int, 3>, ClassPlan> tuned;
 	ClassPlan plan_override[NCLASS];
 	bool override_on[NCLASS] = {};
+	// under an override: the plan that each class's chains ran by (those that
+	// did not speculate), and whether it is the override's
+	ClassPlan ran[NCLASS];
+	bool ran_override[NCLASS] = {};
 	// the user grid (--user_grid): its geometry and corner-packed values
 	struct UserGrid
 	{
@@ -1794,6 +1798,36 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 	auto cost_of = [&](int i) {
 		return double(ch->num_steps[i]) * std::max(1, ch->maxiters[i]) * (b.h.hdr[ch->model[i]].npairs + 1400.0);
 	};
+	// chains per workgroup and form of a size class: a probe's override, else
+	// the tuned plan of the class, where it fits, else the occupancy rule
+	struct Form
+	{
+		int waves, resident;
+		bool persist, tuned;
+	};
+	auto form_of = [&](int ki, const WavePlan& plan, int maxper) {
+		Form f{0, 0, pdef, false};
+		f.waves = occupancy_waves<T, S>(plan, b.precision, variant, pdef, maxper, share, &f.resident);
+		const sgpu_ctx::ClassPlan* cp = nullptr;
+		auto it = c->tuned.find({b.precision, variant, ki});
+		if (c->override_on[ki])
+			cp = &c->plan_override[ki];
+		else if (it != c->tuned.end())
+			cp = &it->second;
+		if (cp && cp->waves >= 1 && cp->waves <= std::min(MAX_CHAINS_PER_GROUP, maxper))
+		{
+			const int bytes = plan_bytes(plan, b.precision, cp->waves);
+			const int per_cu = bytes + LDS_STATIC <= LDS_LIMIT
+					? mc_blocks_per_cu<T, S>(cp->waves, size_t(bytes), variant, cp->persist, false, plan.pair_lds)
+					: 0;
+			if (per_cu > 0)
+				f = {cp->waves, per_cu * maxper / ((maxper + cp->waves - 1) / cp->waves), cp->persist, true};
+		}
+		return f;
+	};
+	int launch_of[sgpu_ctx::NCLASS]; // the class whose launch takes a class's chains
+	for (int k = 0; k < sgpu_ctx::NCLASS; k++)
+		launch_of[k] = k;
 	if (may_speculate && spec == 1 && !forced)
 	{
 		// With more chains than that, the longest may speculate
@@ -1809,10 +1843,11 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 		for (Cls& k : cls)
 			if (!k.members.empty())
 			{
-				int maxper = 1, resident = 0;
+				int maxper = 1;
 				for (auto& kv : k.members)
 					maxper = std::max(maxper, int(kv.second.size()));
-				occupancy_waves<T, S>(plan_for(b.h, k.models()), b.precision, variant, pdef, maxper, share, &resident);
+				const int resident =
+						&k - cls < sgpu_ctx::NCLASS ? form_of(int(&k - cls), plan_for(b.h, k.models()), maxper).resident : 0;
 				for (auto& kv : k.members)
 					for (int i : kv.second)
 					{
@@ -1866,6 +1901,8 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 			{
 				cls[next].members.insert(cls[k].members.begin(), cls[k].members.end());
 				cls[k].members.clear();
+				for (int& l : launch_of)
+					l = l == k ? next : l;
 			}
 		}
 	}
@@ -1925,34 +1962,22 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 		int maxper = 1;
 		for (auto& kv : k.members)
 			maxper = std::max(maxper, int(kv.second.size()));
-		// chains per workgroup by the occupancy rule
-		k.waves = occupancy_waves<T, S>(k.plan, b.precision, variant, pdef, maxper, share, &k.resident);
-		require(k.waves > 0, "chain state exceeds LDS");
-		// a probe's override, else the tuned plan of this class, where it fits
-		const sgpu_ctx::ClassPlan* cp = nullptr;
-		if (ki < sgpu_ctx::NCLASS && c->override_on[ki])
-			cp = &c->plan_override[ki];
-		else if (ki < sgpu_ctx::NCLASS)
-		{
-			auto it = c->tuned.find({b.precision, variant, ki});
-			if (it != c->tuned.end())
-				cp = &it->second;
-		}
 		if (width > 1)
 		{
 			// one chain per workgroup of `width` waves
 			k.waves = width;
 			k.spec = true;
 			k.resident = width * spec_per_cu(k.plan, width);
+			require(k.resident > 0, "chain state exceeds LDS");
 		}
-		else if (cp && cp->waves >= 1 && cp->waves <= std::min(MAX_CHAINS_PER_GROUP, maxper) &&
-				plan_bytes(k.plan, b.precision, cp->waves) + LDS_STATIC <= LDS_LIMIT &&
-				mc_blocks_per_cu<T, S>(cp->waves, size_t(plan_bytes(k.plan, b.precision, cp->waves)), variant,
-						cp->persist, false, k.plan.pair_lds) > 0)
+		else
 		{
-			k.waves = cp->waves;
-			k.persist = cp->persist;
-			k.tuned = true;
+			const Form f = form_of(ki, k.plan, maxper);
+			require(f.waves > 0, "chain state exceeds LDS");
+			k.waves = f.waves;
+			k.resident = f.resident;
+			k.persist = f.persist;
+			k.tuned = f.tuned;
 		}
 		if (std::getenv("SGPU_LOG_PLAN"))
 		{
@@ -2050,7 +2075,6 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 	// device keeps resident at once for its plan; they take the class's
 	// items (costliest first) from a work-queue counter, one counter per
 	// class and part, cleared by a kernel at the start.
-	// the default form unless a tuned plan says otherwise
 	// SGPU_PERSIST_GRID caps a persistent grid's workgroups (each then runs
 	// more items)
 	const char* genv = std::getenv("SGPU_PERSIST_GRID");
@@ -2058,13 +2082,19 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 	for (Cls& k : cls)
 		if (!k.blks.empty())
 		{
-			if (!k.tuned)
-				k.persist = pdef && !k.spec;
 			const int per_cu = mc_blocks_per_cu<T, S>(k.waves, size_t(plan_bytes(k.plan, b.precision, k.waves)),
 					variant, k.persist, k.spec, k.plan.pair_lds);
 			k.grid = k.persist ? std::max(1, std::min({int(k.blks.size()), per_cu * prop.multiProcessorCount, grid_cap}))
 			                   : int(k.blks.size());
 		}
+	// (a launch of speculative chains holds one chain per workgroup)
+	for (int k = 0; k < sgpu_ctx::NCLASS; k++)
+	{
+		const Cls& l = cls[launch_of[k]];
+		const bool own = !l.blks.empty() && !l.spec;
+		c->ran[k] = {own ? l.waves : 1, own && l.persist};
+		c->ran_override[k] = own && launch_of[k] == k && c->override_on[k] && l.tuned;
+	}
 	DBuf dqueue;
 	const int nqueue = NGROUP * (parts + 1);
 	dqueue.alloc(size_t(nqueue) * sizeof(int));
@@ -2267,13 +2297,15 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 	}
 }
 
-// The launch-plan autotuner: for each size class of the request, the
-// class's chains alone run probe_steps Monte Carlo steps from their start
-// state under every candidate plan (chains per workgroup 1, 2, 4, 8 where
-// LDS and the chains per ligand allow; one-shot or persistent grid), timed
-// with HIP events; the fastest plan is kept for the context's later
-// launches of that precision, kernel variant and class.  The chains'
-// trajectories do not depend on the plan, so the probes time the same work.
+// The launch-plan autotuner: every chain runs from its start state, its steps
+// scaled by one factor (the longest chain's to probe_steps), under each
+// candidate plan for all size classes at once, timed with HIP events; the
+// fastest plan is kept for the context's later launches of that precision,
+// kernel variant and class.  The chains' trajectories do not depend on the
+// plan, so the probes time the same work.  A probe is launched as run_mc
+// launches these chains: the longest may speculate, in launches of their own,
+// and a class may join the next one's launch.  The report says what each
+// class's chains ran by, and only a plan that its class ran is kept.
 template<typename T, typename S>
 void run_tune(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, const sgpu_chains* ch,
 		int probe_steps, sgpu_mc_tune_report* rep)
@@ -2400,6 +2432,7 @@ void run_tune(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, c
 	sgpu_chain_results res{maxp, ch->conf_stride, 3 * hmax, cnt.data(), oe.data(), oc.data(), ox.data(), nullptr};
 	double best_ms = 0;
 	int best = 0;
+	std::array<std::array<bool, SGPU_TUNE_MAX_CANDIDATES>, sgpu_ctx::NCLASS> own{}; // the class ran the candidate's plan
 	for (int j = -1; j < int(cands.size()); j++)
 	{
 		// j = -1: an untimed first run (code objects, buffers)
@@ -2416,8 +2449,9 @@ void run_tune(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, c
 		for (int ci = 0; ci < rep->nclasses; ci++)
 		{
 			const int k = rep->class_index[ci];
-			rep->cand_waves[ci][j] = cj.plan[k].waves;
-			rep->cand_persist[ci][j] = cj.plan[k].persist ? 1 : 0;
+			rep->cand_waves[ci][j] = c->ran[k].waves;
+			rep->cand_persist[ci][j] = c->ran[k].persist ? 1 : 0;
+			own[size_t(ci)][size_t(j)] = c->ran_override[k];
 			rep->cand_ms[ci][j] = ms;
 			rep->ncand[ci] = j + 1;
 		}
@@ -2433,9 +2467,14 @@ void run_tune(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, c
 	for (int ci = 0; ci < rep->nclasses; ci++)
 	{
 		const int k = rep->class_index[ci];
-		rep->chosen_waves[ci] = cands[size_t(best)].plan[k].waves;
-		rep->chosen_persist[ci] = cands[size_t(best)].plan[k].persist ? 1 : 0;
-		c->tuned[{b.precision, variant, k}] = cands[size_t(best)].plan[k];
+		rep->chosen_waves[ci] = rep->cand_waves[ci][best];
+		rep->chosen_persist[ci] = rep->cand_persist[ci][best];
+		// the default is no plan of its own: a later launch takes it for its
+		// own number of chains
+		if (best == 0)
+			c->tuned.erase({b.precision, variant, k});
+		else if (own[size_t(ci)][size_t(best)])
+			c->tuned[{b.precision, variant, k}] = cands[size_t(best)].plan[k];
 	}
 }
 

@@ -362,20 +362,26 @@ sgpu_status sgpu_run_mc(sgpu_ctx* ctx, int batch_id, int grid_id, const sgpu_mc_
  * (src/gpu/gpu_kernels_impl.cuh:552-605).  A candidate is one plan for
  * every size class of these chains (by pair count) at once.  The first is
  * the default plan (per class the chains per workgroup with the most
- * resident waves per CU, the larger on ties, and the default form); the
+ * resident chains per CU, the larger on ties but no larger than an even share
+ * of the chains per CU, and the default form); the
  * others take a target of 8, 4, 2 or 1 chains per workgroup (each class
  * the largest count up to the target that its LDS plan and chains per
  * ligand allow) and one form, one-shot grid or persistent grid over a
  * device work queue.  Every chain runs from its start state with its steps
  * scaled by one factor, the longest chain's to probe_steps, under each
  * candidate, the classes concurrently as in a real launch (they share the
- * device, so a class's plan is only good together with the others').  Each
+ * device, so a class's plan is only good together with the others).  Each
  * probe is timed with HIP events.  A candidate replaces the default only
- * when it is more than 3% faster; the chosen plans are kept by the context
- * for its later sgpu_run_mc calls of the same precision, kernel variant
- * and class.  The chains' trajectories do not depend on the plan.  The
- * report lists, per class, its plan under every candidate with the
- * candidate's time, and the choice. */
+ * when it is more than 3% faster; its plans are kept by the context for its
+ * later sgpu_run_mc calls of the same precision, kernel variant and class
+ * (where the default wins, none is, and later calls take their own default).
+ * A plan holds for the chains of its class that run alone: where the longest
+ * chains of a request speculate, they have launches of their own, and a class
+ * may then join the next one's launch.  The chains' trajectories do not
+ * depend on the plan.  The report lists, per class, what its chains ran by
+ * under every candidate (one chain per workgroup where all of them
+ * speculate) with the candidate's time, and the choice; a class that did not
+ * run the chosen candidate's plan in a launch of its own keeps none from it. */
 #define SGPU_TUNE_MAX_CANDIDATES 8
 typedef struct sgpu_mc_tune_report
 {

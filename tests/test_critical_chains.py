@@ -80,3 +80,73 @@ def test_a_very_large_fp64_ligand_beside_smaller_ones(largest, second, monkeypat
     assert any(s for _, _, _, s in plan), plan
     for x, y in zip(a, b):
         assert np.array_equal(x, y)
+
+
+def test_tuner_keeps_only_plans_that_ran(monkeypatch, capfd):
+    """A request of four size classes whose longest chains speculate in
+    launches of their own: the smallest classes join the next one's launch,
+    and the report shows them by that launch's plan; their candidate's plan,
+    which never ran, is not kept.  A small request, whose every chain
+    speculates, keeps none either."""
+    gd, rec = gd_c0(), receptor()
+    shapes = [(10, 2)] * 6 + [(38, 9), (48, 9), (60, 14), (80, 18), (50, 10)]
+    ligs = [sg.Mol.ligand(30 + k, *s) for k, s in enumerate(shapes)]
+    flats = [sg.Flat(m) for m in ligs]
+    size_class = [sum(f.npairs > b for b in (256, 512, 1024)) for f in flats]
+    assert size_class == [0] * 6 + [1, 2, 3, 3, 2]
+    n, smooth, fast = sg.build_tables(sg.vina_scoring())
+    cs, xs = max(f.conf_size for f in flats), 3 * max(f.nheavy for f in flats)
+    monkeypatch.setenv("SGPU_LOG_PLAN", "1")
+
+    def context():
+        ctx = sg.Context(0)
+        ctx.upload_tables(n, smooth, fast)
+        rid = ctx.upload_receptor(rec.xyz, rec.type)
+        return ctx, ctx.build_grids(rid, gd, heavy_types(*ligs), sg.FP32), ctx.upload_models(flats, sg.FP32)
+
+    def request(models):
+        seeds = [flats[m].make_chain(50 + k % 64, gd) for k, m in enumerate(models)]
+        confs = np.zeros((len(models), cs))
+        for k, (c, _) in enumerate(seeds):
+            confs[k, :len(c)] = c
+        # two ligands of many iterations, among them one of class 3 and one of class 2
+        return models, confs, np.array([s for _, s in seeds]), [{9: 24, 10: 30}.get(m, 4) for m in models]
+
+    def plans(text):
+        return [(int(k), int(w), s != "") for k, w, s in re.findall(
+            r"mc class (\d+): \d+ models, (\d+) waves/workgroup( \(one speculative chain\))?,", text)]
+
+    def launches(ctx, gid, bid, models):
+        capfd.readouterr()
+        m, confs, rngs, iters = request(models)
+        ctx.run_mc(bid, gid, sg.mc_params(), m, confs, rngs, [2] * len(m), iters, coord_stride=xs)
+        return plans(capfd.readouterr().err)
+
+    ctx, gid, bid = context()
+    _, cus = ctx.device_info()
+    many = [9] * 8 + [10] * 8 + [m for m in (6, 7, 8) for _ in range(16)] + [k % 6 for k in range(14 * cus - 64)]
+    default = launches(ctx, gid, bid, many)
+    m, confs, rngs, iters = request(many)
+    rep = ctx.tune_mc(bid, gid, sg.mc_params(), m, confs, rngs, iters, probe_steps=2)
+    probes = plans(capfd.readouterr().err)
+    ran = {k for k, _, s in probes if not s}
+    print(default, sorted(set(probes)), rep, flush=True)
+    assert any(s for _, _, s in default) and len(default) <= 4
+    joined = [c for c in rep if c["class"] not in ran]
+    assert [c["class"] for c in rep] == [0, 1, 2, 3] and joined and 3 in ran
+    for c in joined:
+        into = next(d for d in rep if d["class"] > c["class"] and d["class"] in ran)
+        assert c["candidates"] == into["candidates"] and c["chosen"] == into["chosen"]
+    # a request of the smallest ligands alone runs by its default, as before
+    few = [k % 6 for k in range(14 * cus)]
+    tuned = launches(ctx, gid, bid, few)
+    ctx.close()
+    ctx, gid, bid = context()
+    assert launches(ctx, gid, bid, few) == tuned
+    ctx.close()
+    ctx, gid, bid = context()
+    m, confs, rngs, iters = request([0, 1, 6, 7])
+    for c in ctx.tune_mc(bid, gid, sg.mc_params(), m, confs, rngs, iters, probe_steps=2):
+        assert all((x["waves"], x["persistent"]) == (1, False) for x in c["candidates"])
+    assert launches(ctx, gid, bid, many) == default
+    ctx.close()
