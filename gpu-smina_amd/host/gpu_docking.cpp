@@ -5,12 +5,10 @@
  * initial confs must be the exact doubles smina computes.
  */
 #include "gpu_docking.h"
+#include "parallel.h"
 
 #include <algorithm>
 #include <chrono>
-#include <thread>
-#include <system_error>
-#include <exception>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -1264,53 +1262,6 @@ void GpuDocking::fp64_errors(DockJob* const* jobs, size_t nj, int batch, int cst
 			job->fp64_error = std::fabs(job->e_search - job->e_fp64);
 		}
 	}
-}
-
-// f(0) .. f(n - 1) on up to 16 threads (one for small n), in runs of
-// neighbouring indices; the exception of the lowest index that throws is
-// rethrown
-template<typename F>
-static void parallel_for(size_t n, size_t grain, F&& f)
-{
-	const size_t hw = std::max(1u, std::thread::hardware_concurrency());
-	const size_t nt = std::min({size_t(16), hw, n / std::max<size_t>(1, grain)});
-	if (nt < 2)
-	{
-		for (size_t i = 0; i < n; i++)
-			f(i);
-		return;
-	}
-	std::vector<std::exception_ptr> failed(nt);
-	auto part = [&](size_t t) {
-		try
-		{
-			for (size_t i = n * t / nt; i < n * (t + 1) / nt; i++)
-				f(i);
-		}
-		catch (...)
-		{
-			failed[t] = std::current_exception();
-		}
-	};
-	std::vector<std::thread> threads;
-	size_t started = 1;
-	try
-	{
-		for (; started < nt; started++)
-			threads.emplace_back(part, started);
-	}
-	catch (const std::system_error&)
-	{
-		// no more threads: this one takes the parts that have none
-	}
-	part(0);
-	for (size_t t = started; t < nt; t++)
-		part(t);
-	for (std::thread& t : threads)
-		t.join();
-	for (const std::exception_ptr& e : failed)
-		if (e)
-			std::rethrow_exception(e);
 }
 
 void GpuDocking::dock_sub(DockJob* const* jobs, size_t nj, double budget)
