@@ -128,13 +128,17 @@ int DockingServer::submit(int receptor, const sgpu_model_desc* ligand, int exhau
 size_t DockingServer::job_bytes(const Job& j) const
 {
 	// the device memory a job holds while its launch runs: per chain the
-	// state sgpu_run_mc keeps (generator words, the output container of 64
-	// poses with confs and heavy-atom coordinates, the model's coordinates,
-	// in FP64 the pair energies), per job the model blobs and its FP64 copy
+	// state sgpu_run_mc keeps (generator words, the output container of
+	// max(20, num_modes) poses with confs and heavy-atom coordinates, the
+	// model's coordinates, in FP64 the pair energies), the start state it is
+	// made from and the poses packed for their download, per job the model
+	// blobs and its FP64 copy; at least 64 poses a chain, the account's size
+	// when a container held as many
+	const size_t poses = size_t(std::max(64, 2 * std::max(20, s_.dock.num_modes)));
 	const size_t n = size_t(j.ligand->natoms);
 	const size_t real = s_.dock.precision == SGPU_FP64 ? 8 : 4;
 	const size_t conf = 7 + n; // at most one torsion per atom
-	const size_t chain = 4096 + 64 * (8 * conf + real * 3 * n) + real * 3 * n + (real == 8 ? 8 * n * n / 2 : 0);
+	const size_t chain = 4096 + poses * (8 * conf + real * 3 * n) + real * 3 * n + (real == 8 ? 8 * n * n / 2 : 0);
 	const size_t chains = size_t(j.exhaustiveness) * size_t(s_.dock.chain_split > 1 ? s_.dock.chain_split : 1);
 	return chains * chain + 48 * n * n + (1u << 20);
 }

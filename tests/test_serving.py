@@ -143,6 +143,25 @@ def test_device_wide_budget_admits_by_memory():
     del srv
 
 
+@pytest.mark.parametrize("num_modes", [9, 32, 64])
+@pytest.mark.parametrize("prec", [sg.FP32, sg.FP64], ids=["fp32", "fp64"])
+def test_the_account_covers_the_saved_minima_and_their_download(prec, num_modes):
+    """a job's bytes are at least its chains' containers, the same poses
+    packed for their download, and two copies of the generator"""
+    rec = sg.Mol.receptor(11, 400, 8.0)
+    lig = sg.Mol.ligand(720, 14, 2)
+    f = sg.Flat(lig)
+    srv = sg.Server(workers=1, max_batch=1, precision=prec, num_modes=num_modes, step_fraction=1.0 / 4096)
+    r = srv.add_receptor(rec, sg.grid_dims((0.0, 0.0, 0.0), (12.0, 12.0, 12.0)), list(range(2, 14)))
+    chains = 512  # the job's share for its models is under 2 MB
+    srv.wait(srv.submit(r, lig, chains))
+    held = srv.memory()["peak_inflight"]
+    del srv
+    real = 8 if prec == sg.FP64 else 4
+    pose = real * (1 + f.conf_size + 3 * f.nheavy)
+    assert held - 2e6 >= chains * (2 * max(20, num_modes) * pose + 2 * 625 * 4)
+
+
 def test_served_fp64_job_matches_oracle_c4():
     """the serving configuration's sizes: 30 A boxes, receptors of 2,000 and
     6,000 heavy atoms, an 80-heavy-atom ligand with 20 torsions (and a small
