@@ -1578,18 +1578,25 @@ bool persist_default(int variant)
 	return qenv ? std::atoi(qenv) != 0 : mc_private_bytes<T, S>(variant, true) <= mc_private_bytes<T, S>(variant, false);
 }
 
-// the occupancy rule of a size class: chains per workgroup for the most
-// resident chains per CU (registers and LDS, from the runtime's occupancy
-// calculator, less the waves that a ligand's last workgroup leaves empty: 8
-// chains in workgroups of 6 fill 8 of 12), then the larger workgroup, and no
-// larger than `share`, an even share of the launch's chains per CU: larger
-// ones leave CUs empty while the chains of one CU wait for each other; 0 when
-// nothing fits
+// the occupancy rule of a size class: the fewest chains per workgroup that
+// keep nine tenths of the most resident chains per CU (registers and LDS, from
+// the runtime's occupancy calculator, less the waves that a ligand's last
+// workgroup leaves empty: 8 chains in workgroups of 6 fill 8 of 12), and no
+// more than `share`, an even share of the launch's chains per CU; 0 when
+// nothing fits.  Larger workgroups share the staged model's LDS, which counts
+// where LDS holds the chains; past that they only wait: for a CU with room
+// for all their waves, and at the end for their slowest chain.  The largest
+// workgroup of the most resident took 186 ms for 64 ligands of 10-60 heavy
+// atoms x 32 chains in mixed precision and 333 ms for 2,048 ligands of 30 x 8
+// in FP32, this 139 and 298 ms; the screen's Monte Carlo launch at 1/16 of its
+// steps 2,469 and 2,374 ms; a cap of 4 or 2 chains instead took 146 and 144,
+// 331 and 315, 2,375 and 2,653 ms.
 template<typename T, typename S>
 int occupancy_waves(const WavePlan& plan, int precision, int variant, bool persist, int maxper, int share,
 		int* resident)
 {
-	int waves = 0, best = 0;
+	std::array<int, MAX_CHAINS_PER_GROUP + 1> held{};
+	int most = 0, waves = 1;
 	for (int w = 1; w <= std::min({MAX_CHAINS_PER_GROUP, maxper, share}); w++)
 	{
 		const int bytes = plan_bytes(plan, precision, w);
@@ -1597,16 +1604,14 @@ int occupancy_waves(const WavePlan& plan, int precision, int variant, bool persi
 			break;
 		const int per_cu = mc_blocks_per_cu<T, S>(w, size_t(bytes), variant, persist, false, plan.pair_lds);
 		const int groups = (maxper + w - 1) / w;
-		const int r = w * per_cu * maxper / (groups * w);
-		if (r >= best && r > 0)
-		{
-			best = r;
-			waves = w;
-		}
+		held[size_t(w)] = w * per_cu * maxper / (groups * w);
+		most = std::max(most, held[size_t(w)]);
 	}
+	while (most > 0 && 10 * held[size_t(waves)] < 9 * most)
+		waves++;
 	if (resident)
-		*resident = best;
-	return waves;
+		*resident = held[size_t(waves)];
+	return most > 0 ? waves : 0;
 }
 
 // the widths at which single chains of a launch speculate, and what the

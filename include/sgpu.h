@@ -361,9 +361,9 @@ sgpu_status sgpu_run_mc(sgpu_ctx* ctx, int batch_id, int grid_id, const sgpu_mc_
  * whose threads-per-chain policy is a fixed rule
  * (src/gpu/gpu_kernels_impl.cuh:552-605).  A candidate is one plan for
  * every size class of these chains (by pair count) at once.  The first is
- * the default plan (per class the chains per workgroup with the most
- * resident chains per CU, the larger on ties but no larger than an even share
- * of the chains per CU, and the default form); the
+ * the default plan (per class the fewest chains per workgroup within a tenth
+ * of the most resident chains per CU, no more than an even share of the
+ * chains per CU, and the default form); the
  * others take a target of 8, 4, 2 or 1 chains per workgroup (each class
  * the largest count up to the target that its LDS plan and chains per
  * ligand allow) and one form, one-shot grid or persistent grid over a
