@@ -752,9 +752,9 @@ struct ChainState
 	int* ints;        // [0] mt position, [1] pose count, [2] started, [3..3+MAX_POSES) order
 	S* tmp;           // current conf (conf stride)
 	S* scal;          // [0] current e, [1] best e
-	S* out_e;         // [MAX_POSES]
-	S* out_conf;      // [MAX_POSES][conf stride]
-	T* out_coords;    // [MAX_POSES][coord stride]
+	S* out_e;         // [ChainLayout::max_poses]
+	S* out_conf;      // [max_poses][conf stride]
+	T* out_coords;    // [max_poses][coord stride]
 	T* model_coords;  // the model's coordinates (3 * movable) between launches
 	T* root_origin;   // [MAX_TREES * 3]
 	T* pbuf;          // pair-energy scratch (ordered mode)

@@ -42,15 +42,17 @@ namespace sgpu
 
 constexpr int WAVE = 64;
 constexpr int LDS_LIMIT = 160 * 1024; // a workgroup's LDS
-constexpr int MAX_ATOMS = 255;    // movable + fixed atoms per model (8-bit partner field)
-constexpr int MAX_PAIRS = 8191;   // 13-bit pair field
-constexpr int MAX_FRAMES = 64;
-constexpr int MAX_CHANGE = 64;
+// A model's limits: those of the calls' interface, within what the packed
+// records below hold.
+constexpr int MAX_ATOMS = 255;    // movable + fixed atoms (bytes of the pair and frame records)
+constexpr int MAX_PAIRS = 8191;
+constexpr int MAX_FRAMES = 64;    // a lane each; bytes of the atom records and of the paths
+constexpr int MAX_CHANGE = 64;    // a lane per element
 constexpr int MAX_CONF = 64;
 constexpr int MAX_TREES = 16;
-constexpr int MAX_POSES = 64;
-constexpr int MAX_PATH = 32;
-constexpr int MAX_CHAINS_PER_GROUP = 8; // waves of one Monte Carlo workgroup      // frames on a root-to-frame path (ancestor walk of set_conf)
+constexpr int MAX_POSES = 64;     // saved minima of a chain: a lane each
+constexpr int MAX_PATH = 32;      // frames on a root-to-frame path (ancestor walk of set_conf)
+constexpr int MAX_CHAINS_PER_GROUP = 8; // waves of one Monte Carlo workgroup
 
 // conf element kinds: position component, quaternion component a..d, torsion
 enum ConfKind
@@ -68,6 +70,13 @@ enum ChangeKind
 };
 
 constexpr int NBR_BATCH = 4; // codes a neighbour list is padded to
+// The packed fields that a larger limit would overflow: bytes for atoms and
+// frames, 16 bits for a range of neighbour codes (two per pair and a list's
+// padding), and in the FP32 form of a code (search.h) 16 bits each for the
+// byte offsets of an atom's 16 bytes and of a pair's 4.
+static_assert(MAX_ATOMS <= 255 && MAX_FRAMES <= 255 && MAX_CONF <= 255 && MAX_CHANGE <= 255, "bytes of the records");
+static_assert(2 * MAX_PAIRS + (NBR_BATCH - 1) * MAX_ATOMS <= 0xffff, "a neighbour range in an atom's record");
+static_assert(16 * MAX_ATOMS <= 0xffff && 4 * (MAX_PAIRS + 1) <= 0xffff, "byte offsets of a staged neighbour code");
 __host__ __device__ inline int make_code(int partner, int slot) { return int(unsigned(partner) | (unsigned(slot) << 16)); }
 __host__ __device__ inline int code_partner(int c) { return c & 0xffff; }
 __host__ __device__ inline int code_slot(int c) { return int(unsigned(c) >> 16); }

@@ -6,7 +6,7 @@ search: the atom loops and the FP32 prefix scans over two 64-atom chunks
 (with the carry between them), pair loops of many batches and frames past a
 row of 16 lanes.  FP64 evaluation, Monte Carlo and refinement bit-exact
 against the oracle; FP32 within the served tolerance.  A model with more
-pairs than the 13-bit pair field holds is refused with an error."""
+than 8,191 pairs is refused with an error."""
 import numpy as np
 import pytest
 
@@ -87,7 +87,7 @@ def test_large_mc_and_refine_fp64_bit_exact(big):
 
 
 def test_model_past_the_pair_limit_is_refused(big):
-    """150 heavy atoms: 8,904 pairs, past the 8,191 the 13-bit field holds"""
+    """150 heavy atoms: 8,904 pairs, past the limit of 8,191"""
     f = sg.Flat(sg.Mol.ligand(7, 150, 20))
     assert f.npairs > 8191
     with pytest.raises(sg.SgpuError) as err:
