@@ -196,8 +196,8 @@ enum PointTables
 // from LDS) and skip an atom none of them reaches.  A thread per x-fastest
 // point (nine lists a wave, an index, a position and a type load per entry, a
 // gather per ligand type) took 1,676 us for the 531,441 points and 8 types of
-// a 30 A box, this 345 us with all of a cell's tiles in one workgroup (four
-// entries' rows in flight at once: no faster).  With one workgroup a cell, a
+// a 30 A box, this 307 us (345 with all of a cell's tiles in one workgroup;
+// four entries' rows in flight at once: no faster).  With one workgroup a cell, a
 // box of few cells or of many points a cell left most of the device idle: a
 // whole build of a 12 A box at 0.1 A took 4.7 ms (linear) and 40 ms (spline),
 // of a 22.5 A box at 0.375 A with splines 1.77 ms; split, 1.1, 2.6 and 1.27 ms.
