@@ -437,8 +437,7 @@ void pack_batch(const sgpu_flat_model* ms, int n, HostBatch& B)
 				I.push_back(i);
 				++nh;
 			}
-		h.nheavy = nh;
-		h.heavy_lanes = m.natoms > WAVE && nh >= 1 && nh <= WAVE && !hydrogen_pair;
+		h.heavy = nh | (hydrogen_pair || nh == 0 ? ALL_LANES : 0);
 		// trees
 		std::vector<int> troot(m.ntrees, -1), tab(m.ntrees, m.natoms), tae(m.ntrees, 0), tn(m.ntrees, 0);
 		for (int f = 0; f < m.nframes; f++)
@@ -1710,7 +1709,7 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 		require(ch->model[i] >= 0 && ch->model[i] < b.n, "chain model out of range");
 		const ModelHdr& h = b.h.hdr[ch->model[i]];
 		require(ch->conf_stride >= h.conf_size && out->conf_stride >= h.conf_size, "conf stride");
-		require(out->coord_stride >= 3 * h.nheavy, "coord stride");
+		require(out->coord_stride >= 3 * heavy_atoms(h), "coord stride");
 		require(ch->num_steps[i] >= 0 && ch->maxiters[i] >= 0, "steps / maxiters");
 		require(ch->rng[size_t(i) * 625 + 624] <= 624, "rng position");
 		require(!ch->unit || ch->unit[i] >= 0, "search unit");
@@ -1915,7 +1914,7 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 	L.conf_stride = b.h.plan.cmax;
 	int hmax = 1;
 	for (const ModelHdr& h : b.h.hdr)
-		hmax = std::max(hmax, h.nheavy);
+		hmax = std::max(hmax, heavy_atoms(h));
 	L.coord_stride = 3 * hmax;
 	L.atom_stride = 3 * b.h.plan.nmax;
 	L.pair_stride = b.h.plan.pmax;
@@ -2264,10 +2263,10 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 	for (int i = 0; i < n; i++)
 	{
 		const ModelHdr& h = b.h.hdr[ch->model[i]];
-		rows[size_t(i)] = {ne, nc, nx, h.conf_size, 3 * h.nheavy};
+		rows[size_t(i)] = {ne, nc, nx, h.conf_size, 3 * heavy_atoms(h)};
 		ne += size_t(out->count[i]);
 		nc += size_t(out->count[i]) * h.conf_size;
-		nx += size_t(out->count[i]) * 3 * h.nheavy;
+		nx += size_t(out->count[i]) * 3 * heavy_atoms(h);
 	}
 	std::unique_ptr<S[]> pe(new S[std::max<size_t>(1, ne)]), pc(new S[std::max<size_t>(1, nc)]);
 	std::unique_ptr<T[]> px(new T[std::max<size_t>(1, nx)]);
@@ -2324,7 +2323,7 @@ void run_tune(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, c
 	{
 		require(ch->model[i] >= 0 && ch->model[i] < b.n, "chain model out of range");
 		members[mc_class(b.h.hdr[ch->model[i]])].push_back(i);
-		hmax = std::max(hmax, b.h.hdr[ch->model[i]].nheavy);
+		hmax = std::max(hmax, heavy_atoms(b.h.hdr[ch->model[i]]));
 	}
 	hipDeviceProp_t prop;
 	hip_check(hipGetDeviceProperties(&prop, c->device), "hipGetDeviceProperties");
@@ -2497,7 +2496,7 @@ void run_refine(sgpu_ctx* c, const sgpu_refine_request* q)
 		require(q->conf_stride >= b.h.hdr[q->model[i]].conf_size, "conf stride");
 		require(q->maxiters[i] >= 0, "maxiters");
 		if (q->coords)
-			require(q->coord_stride >= 3 * b.h.hdr[q->model[i]].nheavy, "coord stride");
+			require(q->coord_stride >= 3 * heavy_atoms(b.h.hdr[q->model[i]]), "coord stride");
 	}
 	DBuf dboxes;
 	if (q->boxes)
@@ -2525,7 +2524,7 @@ void run_refine(sgpu_ctx* c, const sgpu_refine_request* q)
 	const int cs = b.h.plan.cmax, ps = b.h.plan.pmax;
 	int hmax = 1;
 	for (const ModelHdr& h : b.h.hdr)
-		hmax = std::max(hmax, h.nheavy);
+		hmax = std::max(hmax, heavy_atoms(h));
 	const int xs = 3 * hmax;
 	std::vector<S> conf(size_t(n) * cs, S(0));
 	for (int i = 0; i < n; i++)
@@ -2564,7 +2563,7 @@ void run_refine(sgpu_ctx* c, const sgpu_refine_request* q)
 			q->conf[size_t(i) * q->conf_stride + k] = double(conf[size_t(i) * cs + k]);
 		q->e[i] = e[i] >= Real_host_max<S>() ? DBL_MAX : double(e[i]);
 		if (q->coords)
-			for (int k = 0; k < 3 * h.nheavy; k++)
+			for (int k = 0; k < 3 * heavy_atoms(h); k++)
 				q->coords[size_t(i) * q->coord_stride + k] = double(x[size_t(i) * xs + k]);
 	}
 	if (flag)

@@ -943,7 +943,7 @@ __device__ inline void add_to_output(const MV<T>& m, const WaveMem<T>& W, ChainS
 		S x, S e, double min_rmsd, int max_size, int& count)
 {
 	const int lane = lane_id();
-	const int H = m.h.nheavy;
+	const int H = heavy_atoms(m.h);
 	int* order = s.ints + 3;
 	T rmsd = 0;
 	if (lane < count)

@@ -148,11 +148,10 @@ __host__ __device__ inline int map_index(int w) { return w >> 8; }
 struct ModelHdr
 {
 	int natoms, ninflex, nframes, ntrees, nligands, npairs, nother;
-	int conf_size, change_size, nheavy, nlevels, num_tors;
+	int conf_size, change_size, heavy, nlevels, num_tors; // (heavy: heavy_atoms, ALL_LANES)
 	int path_ok; // every root-to-frame path has at most MAX_PATH frames
 	int ncodes;
 	int one_ligand; // one ligand whose pairs are all those after the other pairs
-	int heavy_lanes; // over 64 movable atoms, 1..64 of them heavy, no hydrogen in a pair (eval_deriv)
 	int iblob_off, iblob_len; // in the batch int blob
 	int tblob_off, tblob_len; // in the batch real blob
 	// offsets inside the int blob (the movable atoms' records at 0)
@@ -160,6 +159,13 @@ struct ModelHdr
 	// offsets inside the real blob
 	int o_xyz0, o_local, o_forig, o_faxis, o_charge;
 };
+
+// ModelHdr::heavy: the movable heavy atoms, and whether every atom takes a lane
+// of the evaluation whatever their number (a pair holds a hydrogen, or there
+// is no heavy atom).  One value for both: the search kernels have no scalar
+// register to spare, and a second one cost a single chain up to 6%.
+constexpr int ALL_LANES = 1 << 16;
+__host__ __device__ inline int heavy_atoms(const ModelHdr& h) { return h.heavy & (ALL_LANES - 1); }
 
 template<typename T>
 struct BatchPtrs

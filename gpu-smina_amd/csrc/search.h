@@ -394,11 +394,10 @@ __device__ inline MV<T> stage_model(const BatchPtrs<T>& B, int m, unsigned char*
 	v.h.nother = own(uniform(h.nother));
 	v.h.conf_size = own(uniform(h.conf_size));
 	v.h.change_size = own(uniform(h.change_size));
-	v.h.nheavy = own(uniform(h.nheavy));
+	v.h.heavy = own(uniform(h.heavy));
 	v.h.nlevels = own(uniform(h.nlevels));
 	v.h.path_ok = own(uniform(h.path_ok));
 	v.h.one_ligand = own(uniform(h.one_ligand));
-	v.h.heavy_lanes = own(uniform(h.heavy_lanes));
 	v.am = reinterpret_cast<const int2*>(li);
 	v.type = li + own(uniform(h.o_type));
 	v.code = li + own(uniform(h.o_code));
@@ -975,9 +974,10 @@ __device__ __forceinline__ T eval_deriv(const MV<T>& m, const EvalCtx<T>& ec, Wa
 	// The lanes take the atoms, or of a model with more than 64 atoms but at
 	// most 64 heavy ones the heavy atoms, so that they pass once over the
 	// atoms, not twice: hydrogens have no receptor term, and no pairs unless
-	// the caller's model lists some (then every atom takes a lane)
-	const bool by_heavy = m.h.heavy_lanes;
-	const int M = by_heavy ? m.h.nheavy : N;
+	// the caller's model lists some (then every atom takes a lane: ALL_LANES
+	// is past any count)
+	const bool by_heavy = N > WAVE && m.h.heavy <= WAVE;
+	const int M = by_heavy ? m.h.heavy : N;
 	// FP64: the first 64 atoms' map cells are fetched now and consumed after
 	// the pairs, which hide the fetch (chains with a CU to themselves)
 	GridSample<T> gs0;
