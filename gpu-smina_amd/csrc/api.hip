@@ -1577,25 +1577,56 @@ bool persist_default(int variant)
 	return qenv ? std::atoi(qenv) != 0 : mc_private_bytes<T, S>(variant, true) <= mc_private_bytes<T, S>(variant, false);
 }
 
-// the occupancy rule of a size class: the fewest chains per workgroup that
-// keep nine tenths of the most resident chains per CU (registers and LDS, from
-// the runtime's occupancy calculator, less the waves that a ligand's last
-// workgroup leaves empty: 8 chains in workgroups of 6 fill 8 of 12), and no
-// more than `share`, an even share of the launch's chains per CU; 0 when
-// nothing fits.  Larger workgroups share the staged model's LDS, which counts
-// where LDS holds the chains; past that they only wait: for a CU with room
-// for all their waves, and at the end for their slowest chain.  The largest
-// workgroup of the most resident took 186 ms for 64 ligands of 10-60 heavy
+// a chain's cost: its steps, the evaluations of a step (about as many per BFGS
+// iteration for every model) and the time of one, 8.1 us + 5.8 ns a pair on a
+// full device
+double chain_cost(const HostBatch& h, const sgpu_chains* ch, int i)
+{
+	return double(ch->num_steps[i]) * std::max(1, ch->maxiters[i]) * (h.hdr[size_t(ch->model[i])].npairs + 1400.0);
+}
+
+// the size class with more than half of the launch's cost (-1: none)
+int main_class(const HostBatch& h, const sgpu_chains* ch)
+{
+	double cost[sgpu_ctx::NCLASS] = {}, total = 0;
+	for (int i = 0; i < ch->nchains; i++)
+	{
+		const double c = chain_cost(h, ch, i);
+		cost[mc_class(h.hdr[size_t(ch->model[i])])] += c;
+		total += c;
+	}
+	for (int k = 0; k < sgpu_ctx::NCLASS; k++)
+		if (2 * cost[k] > total)
+			return k;
+	return -1;
+}
+
+// The occupancy rule of a size class: chains per workgroup by the resident
+// chains per CU (registers and LDS, from the runtime's occupancy calculator,
+// less the waves that a ligand's last workgroup leaves empty: 8 chains in
+// workgroups of 6 fill 8 of 12), and no more than `share`, an even share of
+// the launch's chains per CU; 0 when nothing fits.
+// The fewest that keep nine tenths of the most resident.  A larger workgroup
+// waits for a CU with room for all its waves, and ends with its slowest chain:
+// the largest of the most resident took 186 ms for 64 ligands of 10-60 heavy
 // atoms x 32 chains in mixed precision and 333 ms for 2,048 ligands of 30 x 8
 // in FP32, this 139 and 298 ms; the screen's Monte Carlo launch at 1/16 of its
 // steps 2,469 and 2,374 ms; a cap of 4 or 2 chains instead took 146 and 144,
 // 331 and 315, 2,375 and 2,653 ms.
+// Of a class that LDS bounds (single chains hold less than that) and that is
+// the launch's `main` one, and where the launch does not fill the device
+// (share below the most resident), the largest of the most resident: its
+// workgroups find whole CUs free, and the chains of one ligand share the
+// staged model and the L1's map cells and table rows.  1,024 ligands of 60
+// heavy atoms took 568 ms with 8 chains and 640 with 4, as many resident; 512
+// FP64 chains of a ligand of 24 with QuickVina 2's history 9.8 ms with 2
+// chains and 10.3 with 1.
 template<typename T, typename S>
-int occupancy_waves(const WavePlan& plan, int precision, int variant, bool persist, int maxper, int share,
+int occupancy_waves(const WavePlan& plan, int precision, int variant, bool persist, int maxper, int share, bool main,
 		int* resident)
 {
 	std::array<int, MAX_CHAINS_PER_GROUP + 1> held{};
-	int most = 0, waves = 1;
+	int most = 0, waves = 1, largest = 0;
 	for (int w = 1; w <= std::min({MAX_CHAINS_PER_GROUP, maxper, share}); w++)
 	{
 		const int bytes = plan_bytes(plan, precision, w);
@@ -1604,10 +1635,16 @@ int occupancy_waves(const WavePlan& plan, int precision, int variant, bool persi
 		const int per_cu = mc_blocks_per_cu<T, S>(w, size_t(bytes), variant, persist, false, plan.pair_lds);
 		const int groups = (maxper + w - 1) / w;
 		held[size_t(w)] = w * per_cu * maxper / (groups * w);
-		most = std::max(most, held[size_t(w)]);
+		if (held[size_t(w)] >= most && held[size_t(w)] > 0)
+		{
+			most = held[size_t(w)];
+			largest = w;
+		}
 	}
 	while (most > 0 && 10 * held[size_t(waves)] < 9 * most)
 		waves++;
+	if ((main && waves > 1) || share < most)
+		waves = largest;
 	if (resident)
 		*resident = held[size_t(waves)];
 	return most > 0 ? waves : 0;
@@ -1796,12 +1833,7 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 		}
 	const bool pdef = persist_default<T, S>(variant);
 	const int share = std::max(1, (n + prop.multiProcessorCount - 1) / prop.multiProcessorCount);
-	// a chain's cost: its steps, the evaluations of a step (about as many per
-	// BFGS iteration for every model) and the time of one, 8.1 us + 5.8 ns a
-	// pair on a full device
-	auto cost_of = [&](int i) {
-		return double(ch->num_steps[i]) * std::max(1, ch->maxiters[i]) * (b.h.hdr[ch->model[i]].npairs + 1400.0);
-	};
+	const int main_k = main_class(b.h, ch);
 	// chains per workgroup and form of a size class: a probe's override, else
 	// the tuned plan of the class, where it fits, else the occupancy rule
 	struct Form
@@ -1811,7 +1843,7 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 	};
 	auto form_of = [&](int ki, const WavePlan& plan, int maxper) {
 		Form f{0, 0, pdef, false};
-		f.waves = occupancy_waves<T, S>(plan, b.precision, variant, pdef, maxper, share, &f.resident);
+		f.waves = occupancy_waves<T, S>(plan, b.precision, variant, pdef, maxper, share, ki == main_k, &f.resident);
 		const sgpu_ctx::ClassPlan* cp = nullptr;
 		auto it = c->tuned.find({b.precision, variant, ki});
 		if (c->override_on[ki])
@@ -1855,7 +1887,7 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 				for (auto& kv : k.members)
 					for (int i : kv.second)
 					{
-						pc[size_t(i)].cost = cost_of(i);
+						pc[size_t(i)].cost = chain_cost(b.h, ch, i);
 						pc[size_t(i)].share[0] = 1.0 / std::max(1, resident);
 						for (int q = 0; q < SPEC_WIDTHS; q++)
 							pc[size_t(i)].share[1 + q] = per_cu[q] > 0 ? 1.0 / per_cu[q] : 0;
@@ -2003,7 +2035,7 @@ void run_mc(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, con
 				for (size_t j = s; j < std::min(cs.size(), s + size_t(k.spec ? 1 : k.waves)); j++)
 				{
 					bk.chains.push_back(cs[j]);
-					bk.cost = std::max(bk.cost, cost_of(cs[j]));
+					bk.cost = std::max(bk.cost, chain_cost(b.h, ch, cs[j]));
 				}
 				k.blks.push_back(bk);
 			}
@@ -2391,7 +2423,8 @@ void run_tune(sgpu_ctx* c, int batch_id, int grid_id, const sgpu_mc_params* p, c
 			if (!members[k].empty())
 				d.plan[k] = {occupancy_waves<T, S>(info[k].plan, b.precision, variant, persist_default<T, S>(variant),
 								info[k].maxper,
-								std::max(1, (ch->nchains + prop.multiProcessorCount - 1) / prop.multiProcessorCount), nullptr),
+								std::max(1, (ch->nchains + prop.multiProcessorCount - 1) / prop.multiProcessorCount),
+								k == main_class(b.h, ch), nullptr),
 						persist_default<T, S>(variant)};
 		cands.push_back(d);
 	}

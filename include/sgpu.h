@@ -362,8 +362,10 @@ sgpu_status sgpu_run_mc(sgpu_ctx* ctx, int batch_id, int grid_id, const sgpu_mc_
  * (src/gpu/gpu_kernels_impl.cuh:552-605).  A candidate is one plan for
  * every size class of these chains (by pair count) at once.  The first is
  * the default plan (per class the fewest chains per workgroup within a tenth
- * of the most resident chains per CU, no more than an even share of the
- * chains per CU, and the default form); the
+ * of the most resident chains per CU, or the largest of the most resident
+ * where the launch does not fill the device or the class is most of it and
+ * bound by LDS, no more than an even share of the chains per CU, and the
+ * default form); the
  * others take a target of 8, 4, 2 or 1 chains per workgroup (each class
  * the largest count up to the target that its LDS plan and chains per
  * ligand allow) and one form, one-shot grid or persistent grid over a

@@ -165,3 +165,33 @@ def test_the_default_workgroups_are_near_the_best():
     ms = [c["ms"] for c in d.tune(ligs, probe_steps=64)[0]["candidates"]]
     print(ms, flush=True)
     assert ms[0] <= 1.15 * min(ms), ms
+
+
+def test_workgroups_of_a_class_that_lds_bounds(monkeypatch, capfd):
+    """a ligand of 66 heavy atoms, whose single chains hold fewer of a CU than
+    workgroups do: alone it takes the largest workgroup of the most resident,
+    among other ligands of more work the smallest that keeps them; a request
+    that does not fill the device takes the largest, too"""
+    ligs = [sg.Mol.ligand(67, 66, 14), sg.Mol.ligand(30, 10, 2)]
+    monkeypatch.setenv("SGPU_SPEC", "1")
+    waves = []
+    for models in ([0] * 2304, [0] * 768 + [1] * 4608, [0] * 512):
+        flats = [sg.Flat(m) for m in ligs]
+        ctx = sg.Context(0)
+        n, smooth, fast = sg.build_tables(sg.vina_scoring())
+        ctx.upload_tables(n, smooth, fast)
+        rid = ctx.upload_receptor(receptor().xyz, receptor().type)
+        gd = gd_c0()
+        gid = ctx.build_grids(rid, gd, heavy_types(*ligs), sg.FP32)
+        bid = ctx.upload_models(flats, sg.FP32)
+        seeds = [[f.make_chain(50 + k, gd) for k in range(8)] for f in flats]
+        confs = np.zeros((len(models), max(f.conf_size for f in flats)))
+        for k, m in enumerate(models):
+            confs[k, :flats[m].conf_size] = seeds[m][k % 8][0]
+        monkeypatch.setenv("SGPU_LOG_PLAN", "1")
+        ctx.run_mc(bid, gid, sg.mc_params(), models, confs, np.array([seeds[m][k % 8][1] for k, m in enumerate(models)]),
+                   [1] * len(models), [5] * len(models), coord_stride=3 * max(f.nheavy for f in flats))
+        ctx.close()
+        waves.append(int(re.search(r"mc class 3: \d+ models, (\d+) waves/workgroup,", capfd.readouterr().err).group(1)))
+    print(waves, flush=True)
+    assert waves[0] > waves[1] and waves[2] == 2, waves
